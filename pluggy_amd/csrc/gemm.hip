@@ -2,6 +2,7 @@
 #include <mutex>
 
 #include "gemm_persist.h"
+#include "gemm_pingpong.h"
 #include "kernels.h"
 
 namespace pmoe {
@@ -17,20 +18,23 @@ template <typename T> struct CfgFor;
 template <> struct CfgFor<bf16_t> { typedef CfgBf16 type; };
 template <> struct CfgFor<float> { typedef CfgF32 type; };
 
-// bf16 expert GEMMs run on the persistent DMA engine: 256x256 blocks of eight
-// 128x64 wave tiles (two waves per SIMD, one block per CU) with a four-stage
-// ring of 32-deep k tiles (128 KiB of LDS) and 16-row epilogue slabs (8-row
-// for fp32 staging). Chosen by measurement at the Qwen3-30B-A3B shape over
-// 128x128 .. 256x256 tilings, 2..5 stages and 32/64-deep k tiles: larger
+// The weight gradients run on the persistent DMA engine: 256x256 blocks of
+// eight 128x64 wave tiles (two waves per SIMD, one block per CU) with a
+// four-stage ring of 32-deep k tiles (128 KiB of LDS) and 16-row epilogue slabs
+// (8-row for fp32 staging). Chosen by measurement at the Qwen3-30B-A3B shape
+// over 128x128 .. 256x256 tilings, 2..5 stages and 32/64-deep k tiles: larger
 // tiles fetch fewer bytes per MFMA through each CU's vector-memory path, which
 // bounds the smaller ones. A fourth stage does not speed up the k-loop, but
 // the next tile's first three stages are then in flight before a tile's
-// epilogue stores, which drain while they are used. Against three stages
-// (with 128 x 512 tiles covering short last m-tiles in the forward GEMMs,
-// whose 40 KiB slots fit only three), same bits, alternating runs on one box:
-// the config-2 step -0.4 to -0.8 % on two boxes (down dgrad -2 %, the other
-// GEMMs within +-1 %), config 3 -0.8 %, config 4 +0.5 % (its many short last
-// m-tiles: gate_up fwd +3 %, down fwd -5 %); fp32 weight gradients the same.
+// epilogue stores, which drain while they are used. The row-grouped GEMMs
+// (forward and input gradients) take the same tiles in the ping-pong loop of
+// gemm_pingpong.h: on this engine's loop they measured, alternating launches
+// at 8192 tokens, gate_up 507 against 472 us, down 289 / 262, down's input
+// gradient 306 / 280, gate_up's 472 / 430; at the Qwen3-235B-A22B layer and
+// 16384 tokens 3270 / 3050, 1674 / 1560, 1801 / 1610, 3022 / 2810. The weight
+// gradients measured the same in that loop (443 / 442 us and 235 / 234; under
+// skewed routing slower), whose 128-byte pieces they have anyway ([k][r]
+// operands: 512-byte ones), so they stay here.
 typedef DmaCfg<256, 256, 128, 64, 4, 32, 1> DmaExpert;
 // Row-grouped GEMMs whose 256-row tiles would leave whole rounds of the
 // persistent walk idle: 128 x 256 blocks of eight 64 x 64 wave tiles (same
@@ -125,7 +129,9 @@ hipError_t expert_gemm_run(int kind, const T* A, const T* B, const T* aux, T* C,
     if (rows == Cfgs::Rows128::BM)
       return expert_gemm_persist_rows<typename Cfgs::Rows128>(kind, A, B, aux, C, C2, offs, P, E, H, I, xg, num_cus(),
                                                                s);
-    return expert_gemm_persist<typename Cfgs::Main, Tw>(kind, A, B, aux, C, C2, Cw, offs, P, E, H, I, xg, num_cus(), s);
+    if (!wgrad)
+      return expert_gemm_pp_rows<PpCfg<T>>(kind, A, B, aux, C, C2, offs, P, E, H, I, xg, num_cus(), s);
+    return expert_gemm_persist_wgrad<typename Cfgs::Main, Tw>(kind, A, B, Cw, offs, P, E, H, I, xg, num_cus(), s);
   } else {
     static_assert(std::is_same<T, Tw>::value, "fp32 operands give fp32 weight gradients");
     return expert_gemm<typename CfgFor<T>::type, T>(kind, A, B, aux, wgrad ? Cw : C, C2, offs, P, E, H, I, xg, s);

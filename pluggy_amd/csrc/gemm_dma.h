@@ -54,6 +54,13 @@ struct DmaCfg {
   static constexpr int EPI_BYTES = NW * 32 * EPI_LD * 4;
   static constexpr int MAIN_BYTES = NS * STAGE_BYTES;
   static constexpr int SMEM_BYTES = MAIN_BYTES > EPI_BYTES ? MAIN_BYTES : EPI_BYTES;
+  // Rows of wave wm's 32-row blocks, relative to the tile: block i starts at
+  // wave_row(wm) + row_blk(i); a wave's rows span ROW_SPAN rows.
+  static constexpr int ROW_SPAN = WM;
+  __device__ static constexpr int wave_row(int wm) { return wm * WM; }
+  __device__ static constexpr int row_blk(int i) { return i * 32; }
+  // 32-deep stages that a GM_RED tile over `rows` reduction rows runs
+  __device__ static __forceinline__ int red_stages(int rows) { return max((rows + BK - 1) / BK, NS - 1) * BK / 32; }
   static_assert(WM % 32 == 0 && WN % 32 == 0 && BM % WM == 0 && BN % WN == 0, "tile shape");
   static_assert(BK == 32 || BK == 64 || BK == 128, "k extent of a stage");
   static_assert(A_INSTR * NW * 1024 == A_BYTES && B_INSTR * NW * 1024 == B_BYTES,
@@ -92,21 +99,24 @@ __device__ __forceinline__ uint32_t lds_addr(const char* p) {
 // compiler adds no waits of its own; every consumer waits explicitly with
 // wait_vmcnt<> and a barrier. m0 (the LDS destination) is an input operand
 // of the statement, so the compiler sets it (often computing the address
-// straight into m0) and knows what it holds. NTL: a non-temporal (streaming)
+// straight into m0) and knows what it holds. The compiler does not look inside
+// the statement for hazards, and the descriptor may reach it straight from a
+// v_readlane (a spilled SGPR), which needs five wait states before a vector
+// memory instruction reads it: hence the s_nop (m0 alone would need one). NTL: a non-temporal (streaming)
 // load, for data each tile reads once and no other tile reuses (the weight
 // stream of the decode tiles).
 template <bool NTL = false>
 __device__ __forceinline__ void dma16(const BufRsrc& rs, uint32_t lds, uint32_t voff) {
   if constexpr (NTL)
     asm volatile(
-        "s_nop 0\n\t"
+        "s_nop 4\n\t"
         "buffer_load_dwordx4 %0, %1, 0 offen nt lds"
         :
         : "v"(voff), "s"(rs), "{m0}"(lds)
         : "memory");
   else
     asm volatile(
-        "s_nop 0\n\t"
+        "s_nop 4\n\t"
         "buffer_load_dwordx4 %0, %1, 0 offen lds"
         :
         : "v"(voff), "s"(rs), "{m0}"(lds)

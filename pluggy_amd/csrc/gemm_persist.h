@@ -118,8 +118,8 @@ __device__ __forceinline__ void stage_get8(const float* stage, int row, int c, f
 template <class Cfg, typename Tout, int GM, bool NT>
 __device__ __forceinline__ void store_tile_full_cols(const f32x16 (&acc)[Cfg::MI][Cfg::NI], float* stage,
                                                      const TileInfo& ti, const GemmParams& p, int wm, int wn,
-                                                     int lane) {
-  constexpr int MI = Cfg::MI, NI = Cfg::NI, WM = Cfg::WM, WN = Cfg::WN;
+                                                     int lane, int blocks) {
+  constexpr int MI = Cfg::MI, NI = Cfg::NI, WN = Cfg::WN;
   constexpr int CPR = WN / 8;  // 8-output chunks per row
   static_assert(PersistLayout<Cfg>::EPI_LD >= 64, "the staged rows hold 64 floats");
   static_assert(8 * CPR == kWave, "one chunk per lane per 8-row slab (64-column wave tiles)");
@@ -127,8 +127,8 @@ __device__ __forceinline__ void store_tile_full_cols(const f32x16 (&acc)[Cfg::MI
   if constexpr (GM == GM_RED) C += (int64_t)ti.group * p.strideC;
   // uniform by construction; said so, or the descriptor lives in VGPRs and
   // every buffer access becomes a readfirstlane loop
-  const int row0 = __builtin_amdgcn_readfirstlane(ti.m0 + wm * WM);
-  const int rows = __builtin_amdgcn_readfirstlane(min(max(ti.m_end - row0, 0), WM));
+  const int row0 = __builtin_amdgcn_readfirstlane(ti.m0 + Cfg::wave_row(wm));
+  const int rows = __builtin_amdgcn_readfirstlane(min(max(ti.m_end - row0, 0), Cfg::ROW_SPAN));
   Tout* base = C + (int64_t)row0 * p.ldc + ti.n0 + wn * WN;
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
       base, (short)0, rows > 0 ? (int)(((int64_t)(rows - 1) * p.ldc + WN) * (int64_t)sizeof(Tout)) : 0, 0x00020000);
@@ -138,6 +138,7 @@ __device__ __forceinline__ void store_tile_full_cols(const f32x16 (&acc)[Cfg::MI
   constexpr int AUX = NT ? 2 : 0;  // nt
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
+    if (i >= blocks) break;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -146,7 +147,7 @@ __device__ __forceinline__ void store_tile_full_cols(const f32x16 (&acc)[Cfg::MI
         for (int rr = 0; rr < 4; ++rr) stage_put(stage, 4 * half + rr, j * 32 + col_l, acc[i][j][4 * q + rr]);
       float v[8];
       stage_get8(stage, r, c, v);
-      const int off = (i * 32 + 8 * q + r) * ld_bytes + c * (int)sizeof(Tout);
+      const int off = (Cfg::row_blk(i) + 8 * q + r) * ld_bytes + c * (int)sizeof(Tout);
       if constexpr (sizeof(Tout) == 2) {
         __builtin_amdgcn_raw_buffer_store_b128(Out8<Tout>::pack(v), rs, off, 0, AUX);
       } else {
@@ -175,14 +176,14 @@ __device__ __forceinline__ void store_tile_full_cols(const f32x16 (&acc)[Cfg::MI
 template <class Cfg, bool NT>
 __device__ __forceinline__ void store_tile_swiglu_bwd(const f32x16 (&acc)[Cfg::MI][Cfg::NI], float* stage,
                                                       const TileInfo& ti, const GemmParams& p, int wm, int wn,
-                                                      int lane) {
-  constexpr int MI = Cfg::MI, NI = Cfg::NI, WM = Cfg::WM, WN = Cfg::WN;
+                                                      int lane, int blocks) {
+  constexpr int MI = Cfg::MI, NI = Cfg::NI, WN = Cfg::WN;
   constexpr int CPR = WN / 8;
   typedef typename Cfg::Tc T16;
   static_assert(WN == 64 && 8 * CPR == kWave, "one 8-column chunk per lane per 8-row slab, 64-column partials");
   constexpr int NSLAB = MI * 4, PF = 2;  // slabs per wave, slabs loaded ahead
-  const int row0 = __builtin_amdgcn_readfirstlane(ti.m0 + wm * WM);  // uniform: scalar descriptors
-  const int rows = __builtin_amdgcn_readfirstlane(min(max(ti.m_end - row0, 0), WM));
+  const int row0 = __builtin_amdgcn_readfirstlane(ti.m0 + Cfg::wave_row(wm));  // uniform: scalar descriptors
+  const int rows = __builtin_amdgcn_readfirstlane(min(max(ti.m_end - row0, 0), Cfg::ROW_SPAN));
   const int col0 = __builtin_amdgcn_readfirstlane(ti.n0 + wn * WN);
   const int r = lane / CPR, c = (lane % CPR) * 8;
   const int ldaux = (int)p.ldaux, ldc = (int)p.ldc;
@@ -201,13 +202,13 @@ __device__ __forceinline__ void store_tile_swiglu_bwd(const f32x16 (&acc)[Cfg::M
   const int half = lane >> 5, col_l = lane & 31;
   u32x4 pg[PF], pu[PF];
   float pw[PF];
-  // slab s: rows 32 (s / 4) + 8 (s % 4) .. +7 of the wave; this lane's row in it is r
+  // slab s: rows 8 (s % 4) .. +7 of the wave's block s / 4; this lane's row in it is r
   // per-lane offsets are fixed; the slab's first row and the column block go
   // in the uniform (SGPR) offset, so the unrolled slabs share four VGPRs
   const int vo_gu = (r * ldaux + c) * 2, vo_dg = (r * ldc + c) * 2, vo_w = r * 4, vo_part = r * p.part_ld * 4;
   auto fetch = [&](auto sc) {
     constexpr int S = decltype(sc)::value;
-    constexpr int R0 = (S / 4) * 32 + 8 * (S % 4);
+    constexpr int R0 = Cfg::row_blk(S / 4) + 8 * (S % 4);
     const int so = (R0 * ldaux + col0) * 2;
     pg[S % PF] = __builtin_amdgcn_raw_buffer_load_b128(rs_gu, vo_gu, so, 0);
     pu[S % PF] = __builtin_amdgcn_raw_buffer_load_b128(rs_gu, vo_gu, so + (int)p.inter * 2, 0);
@@ -216,6 +217,7 @@ __device__ __forceinline__ void store_tile_swiglu_bwd(const f32x16 (&acc)[Cfg::M
   static_for<0, PF>([&](auto sc) { fetch(sc); });
   static_for<0, NSLAB>([&](auto sc) {
     constexpr int S = decltype(sc)::value, i = S / 4, q = S % 4;
+    if (i >= blocks) return;
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
@@ -236,7 +238,7 @@ __device__ __forceinline__ void store_tile_swiglu_bwd(const f32x16 (&acc)[Cfg::M
       dg[t] = dm * u[t] * (sg + silu * (1.0f - sg));
       du[t] = dm * silu;
     }
-    constexpr int R0 = i * 32 + 8 * q;
+    constexpr int R0 = Cfg::row_blk(i) + 8 * q;
     const int so = (R0 * ldc + col0) * 2;
     __builtin_amdgcn_raw_buffer_store_b128(Out8<T16>::pack(dg), rs_dg, vo_dg, so, AUX);
     __builtin_amdgcn_raw_buffer_store_b128(Out8<T16>::pack(du), rs_dg, vo_dg, so + (int)p.inter * 2, AUX);
@@ -251,9 +253,12 @@ __device__ __forceinline__ void store_tile_swiglu_bwd(const f32x16 (&acc)[Cfg::M
   });
 }
 
+// Epilogue of one tile. blocks: the wave's 32-row blocks to store (fewer than
+// MI where the tile has no rows in the others).
 template <class Cfg, typename Tout, int GM, int EPI, bool PACK, int SLAB>
 __device__ __forceinline__ void store_slabs(const f32x16 (&acc)[Cfg::MI][Cfg::NI], float* stage,
-                                            const TileInfo& ti, const GemmParams& p, int wm, int wn, int lane) {
+                                            const TileInfo& ti, const GemmParams& p, int wm, int wn, int lane,
+                                            int blocks = Cfg::MI) {
   constexpr int MI = Cfg::MI, NI = Cfg::NI, WN = Cfg::WN;
   constexpr int LD = PersistLayout<Cfg>::EPI_LD;
   constexpr int LDW = EpiStage<Cfg, PACK, SLAB>::ROW;  // packed: words per staged row
@@ -262,15 +267,15 @@ __device__ __forceinline__ void store_slabs(const f32x16 (&acc)[Cfg::MI][Cfg::NI
   static_assert(EPI == EPI_STORE || sizeof(Tout) == 2, "fused epilogues write bf16");
   constexpr bool NT = nt_epilogue<GM>();
   if constexpr (EPI == EPI_SWIGLU_BWD && GM == GM_ROWS && Cfg::WN == 64) {
-    if (ti.n0 + Cfg::BN <= p.N && (int64_t)Cfg::WM * p.ldaux * 2 < ((int64_t)1 << 31) &&
-        (int64_t)Cfg::WM * p.ldc * 2 < ((int64_t)1 << 31)) {
-      store_tile_swiglu_bwd<Cfg, NT>(acc, stage, ti, p, wm, wn, lane);
+    if (ti.n0 + Cfg::BN <= p.N && (int64_t)Cfg::ROW_SPAN * p.ldaux * 2 < ((int64_t)1 << 31) &&
+        (int64_t)Cfg::ROW_SPAN * p.ldc * 2 < ((int64_t)1 << 31)) {
+      store_tile_swiglu_bwd<Cfg, NT>(acc, stage, ti, p, wm, wn, lane, blocks);
       return;
     }
   }
   if constexpr (EPI == EPI_STORE && Cfg::WN == 64) {
-    if (ti.n0 + Cfg::BN <= p.N && (int64_t)Cfg::WM * p.ldc * (int64_t)sizeof(Tout) < ((int64_t)1 << 31)) {
-      store_tile_full_cols<Cfg, Tout, GM, NT>(acc, stage, ti, p, wm, wn, lane);
+    if (ti.n0 + Cfg::BN <= p.N && (int64_t)Cfg::ROW_SPAN * p.ldc * (int64_t)sizeof(Tout) < ((int64_t)1 << 31)) {
+      store_tile_full_cols<Cfg, Tout, GM, NT>(acc, stage, ti, p, wm, wn, lane, blocks);
       return;
     }
   }
@@ -290,12 +295,13 @@ __device__ __forceinline__ void store_slabs(const f32x16 (&acc)[Cfg::MI][Cfg::NI
 #pragma unroll
         for (int ei = 0; ei < SW_NE; ++ei) {
           const int e = lane + 64 * ei;
-          const int row = ti.m0 + wm * Cfg::WM + i * 32 + SLAB * hs + e / SW_CPR;
+          const int row = ti.m0 + Cfg::wave_row(wm) + Cfg::row_blk(i) + SLAB * hs + e / SW_CPR;
           wsp[i][hs][ei] = (p.row_w != nullptr && e < SLAB * SW_CPR && row < ti.m_end) ? p.row_w[row] : 1.0f;
         }
   }
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
+    if (i >= blocks) break;
 #pragma unroll
     for (int hs = 0; hs < NSL; ++hs) {
       if constexpr (PACK) {
@@ -324,7 +330,7 @@ __device__ __forceinline__ void store_slabs(const f32x16 (&acc)[Cfg::MI][Cfg::NI
       }
       __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0): slab written
       asm volatile("" ::: "memory");
-      const int row_base = ti.m0 + wm * Cfg::WM + i * 32 + SLAB * hs;
+      const int row_base = ti.m0 + Cfg::wave_row(wm) + Cfg::row_blk(i) + SLAB * hs;
       if constexpr (EPI == EPI_SWIGLU) {
         constexpr int H2 = WN / 2, CPR = H2 / 8;
         Tout* MID = reinterpret_cast<Tout*>(p.C2);
@@ -449,13 +455,13 @@ __device__ __forceinline__ void rows_tile(int local, int r, int ntn, int mb, int
   mt = m0 + local % h;
 }
 
-// GM_RED cost model: a tile of group g runs max(ceil(rows_g / BK), NS - 1)
+// GM_RED cost model: a tile of group g runs Cfg::red_stages(rows_g) (32-deep)
 // k-stages plus an epilogue worth about kRedEpiStages stages (measured: a
 // 256x256 bf16 tile drains in ~3 stage times). s_cost[g] = cost of one tile of
 // each group before g (inclusive scan to groups + 1 entries, computed by wave
 // 0), *s_cmax = the largest cost of one tile; every thread gets s_cost[groups].
 constexpr int kRedEpiStages = 3;
-template <int BK, int NS>
+template <class Cfg>
 __device__ __forceinline__ int red_cost_scan(const int32_t* offs, int groups, int* s_cost, int* s_cmax) {
   const int tid = threadIdx.x, lane = tid & 63;
   if (tid < 64) {
@@ -465,7 +471,7 @@ __device__ __forceinline__ int red_cost_scan(const int32_t* offs, int groups, in
       int c = 0;
       if (g < groups) {
         const int rows = offs[g] - (g == 0 ? 0 : offs[g - 1]);
-        c = max((rows + BK - 1) / BK, NS - 1) + kRedEpiStages;
+        c = Cfg::red_stages(rows) + kRedEpiStages;
       }
       cmax = max(cmax, c);
       const int inc = wave_incl_scan(c, lane) + carry;
@@ -572,6 +578,104 @@ __device__ __forceinline__ bool deal_below_mean(const unsigned short* s_order, i
   return s_result[1] == 0 && j0 >= total;
 }
 
+// The tile list of a persistent kernel and this block's tiles of it.
+//
+// XCD x (blocks with blockIdx % 8 == x) takes a contiguous share of the tiles
+// and its blocks walk it in a stride of their count. GM_ROWS tiles all run
+// the full reduction, so the shares hold equal tile counts; a GM_RED tile
+// runs its group's reduction range, so there the shares hold equal cost.
+// Under skewed routing (GM_RED, one tile costing more than half a block's
+// mean share) the shares cannot balance: a heavy group's tiles crowd one
+// XCD's blocks. Then the tiles are taken in order of descending cost and
+// dealt in rounds to the blocks still below the mean share
+// (deal_below_mean), positions XCD-major so that a group's tiles still run
+// side by side on one XCD; when that deal does not fit its bounds, in a
+// snake (round k gives tile k*NB + p to the block at position p, or
+// k*NB + NB-1-p for odd k).
+template <class Cfg, int GM>
+struct TileWalk {
+  int ntiles_n, mt_red;  // n-tiles; GM_RED: m-tiles per group
+  int mb;                // GM_ROWS: m-tiles per super-block of a row-heavy expert (rows_tile)
+  int total, cnt, start, tpg, spos, bi, nb;
+  bool skew;
+  const int* scan;
+  const unsigned short* order;
+
+  // Reads the offsets into s_offs (offs null: one group of all M rows, a plain
+  // GEMM on the same engine), scans them and finds this block's share. Every
+  // thread calls it; false when there is no tile at all for this block. cols /
+  // tile_cols: output columns and those of one tile. scratch: LDS not in use
+  // yet (the ring).
+  __device__ __forceinline__ bool init(const GemmParams& p, int cols, int tile_cols, int* s_offs, int* s_scan,
+                                       unsigned short* s_order, int* s_cmax, int* s_deal, char* scratch) {
+    constexpr int BM = Cfg::BM, NT = Cfg::NT;
+    const int tid = threadIdx.x, groups = p.groups;
+    scan = s_scan;
+    order = s_order;
+    for (int g = tid; g < groups; g += NT) s_offs[g] = p.offs != nullptr ? p.offs[g] : p.M;
+    __syncthreads();
+    ntiles_n = (cols + tile_cols - 1) / tile_cols;
+    mt_red = (p.M + BM - 1) / BM;
+    if constexpr (GM == GM_ROWS) total = rows_scan<BM>(s_offs, groups, s_scan) * ntiles_n;
+    else total = groups * mt_red * ntiles_n;
+    const int xcd = blockIdx.x & 7;
+    nb = ((int)gridDim.x - xcd + 7) >> 3;  // blocks on this XCD
+    bi = blockIdx.x >> 3;                  // this block's position on its XCD
+    // the same for every block (the tile list must be), from the grid's blocks per XCD
+    mb = max(1, ((int)gridDim.x >> 3) / ntiles_n);
+    cnt = 0; start = 0; tpg = 1; spos = 0;
+    skew = false;
+    if (total == 0) return false;
+    if constexpr (GM == GM_RED) {
+      tpg = mt_red * ntiles_n;  // tiles per group
+      const int64_t c_all = red_cost_scan<Cfg>(s_offs, groups, s_scan, s_cmax) * (int64_t)tpg;
+      skew = (int64_t)*s_cmax * 2 * gridDim.x > c_all;
+      if (skew) {
+        for (int g = tid; g < groups; g += NT) {
+          const int c = s_scan[g + 1] - s_scan[g];
+          int r = 0;
+          for (int h = 0; h < groups; ++h) {
+            const int ch = s_scan[h + 1] - s_scan[h];
+            r += (ch > c || (ch == c && h < g)) ? 1 : 0;
+          }
+          s_order[r] = g;
+        }
+        __syncthreads();
+        for (int x = 0; x < xcd; ++x) spos += ((int)gridDim.x - x + 7) >> 3;
+        spos += bi;
+        // spos < 0 from here on: this block's tiles are the list in s_scan
+        if (deal_below_mean<NT>(s_order, s_scan, groups, tpg, total, c_all, (int)gridDim.x, spos, scratch, s_deal))
+          spos = -1;
+      } else {
+        const int b0 = red_cost_tile(s_scan, groups, tpg, c_all * xcd / 8);
+        const int b1 = xcd == 7 ? total : red_cost_tile(s_scan, groups, tpg, c_all * (xcd + 1) / 8);
+        start = b0;
+        cnt = b1 - b0;
+      }
+    } else {
+      const int per = total >> 3, rem = total & 7;
+      cnt = per + (xcd < rem ? 1 : 0);
+      start = xcd * per + (xcd < rem ? xcd : rem);
+    }
+    return at(0) >= 0;
+  }
+
+  // The k-th tile of this block (k = 0, 1, ...) as a list index, or -1 past its last.
+  __device__ __forceinline__ int at(int k) const {
+    if (skew) {
+      if (spos < 0) {
+        const int j = k < kMaxDealt ? scan[k] : -1;  // this block's k-th tile in the cost order
+        return j < 0 ? -1 : order[j / tpg] * tpg + j % tpg;
+      }
+      const int NB = (int)gridDim.x;
+      const int j = k * NB + ((k & 1) ? NB - 1 - spos : spos);
+      return j < total ? order[j / tpg] * tpg + j % tpg : -1;
+    }
+    const int b = bi + k * nb;
+    return b < cnt ? start + b : -1;
+  }
+};
+
 // The block's tiles form one continuous stream of k-stages: stage g lives in
 // ring slot g % NS, and the DMAs issued during stage g fetch stream stage
 // g + NS - 1, which in a tile's last NS - 1 stages is one of the next tile's
@@ -637,83 +741,12 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_persist_kernel(GemmPa
   const int wm = wave / Cfg::WAVES_N, wn = wave % Cfg::WAVES_N;
   const int groups = p.groups;
 
-  // ---- tile list: GM_ROWS m-tiles follow the per-group row counts
-  // offs null: one group of all M rows (a plain GEMM on the same engine)
-  for (int g = tid; g < groups; g += Cfg::NT) s_offs[g] = p.offs != nullptr ? p.offs[g] : p.M;
-  __syncthreads();
-  const int ntiles_n = (EPI == EPI_SWIGLU) ? (p.inter + BN / 2 - 1) / (BN / 2) : (p.N + BN - 1) / BN;
-  const int mt_red = (p.M + BM - 1) / BM;  // GM_RED: m-tiles per group
-  int total;
-  if constexpr (GM == GM_ROWS) total = rows_scan<BM>(s_offs, groups, s_scan) * ntiles_n;
-  else total = groups * mt_red * ntiles_n;
-  // XCD x (blocks with blockIdx % 8 == x) takes a contiguous share of the tiles
-  // and its blocks walk it in a stride of their count. GM_ROWS tiles all run
-  // the full reduction, so the shares hold equal tile counts; a GM_RED tile
-  // runs its group's reduction range, so there the shares hold equal cost.
-  // Under skewed routing (GM_RED, one tile costing more than half a block's
-  // mean share) the shares cannot balance: a heavy group's tiles crowd one
-  // XCD's blocks. Then the tiles are taken in order of descending cost and
-  // dealt in rounds to the blocks still below the mean share
-  // (deal_below_mean), positions XCD-major so that a group's tiles still run
-  // side by side on one XCD; when that deal does not fit its bounds, in a
-  // snake (round k gives tile k*NB + p to the block at position p, or
-  // k*NB + NB-1-p for odd k).
-  const int xcd = blockIdx.x & 7;
-  const int nb = ((int)gridDim.x - xcd + 7) >> 3;  // blocks on this XCD
-  const int bi = blockIdx.x >> 3;                  // this block's position on its XCD
-  // m-tiles per super-block of a row-heavy expert: the same for every block
-  // (the tile list must be), from the grid's blocks per XCD
-  const int mb = max(1, ((int)gridDim.x >> 3) / ntiles_n);
-  int cnt = 0, start = 0, tpg = 1, spos = 0;
-  bool skew = false;
-  if (total == 0) {
+  TileWalk<Cfg, GM> walk;
+  if (!walk.init(p, (EPI == EPI_SWIGLU) ? p.inter : p.N, (EPI == EPI_SWIGLU) ? BN / 2 : BN, s_offs, s_scan, s_order,
+                 &s_cmax, s_deal, smem))
     return;
-  } else if constexpr (GM == GM_RED) {
-    tpg = mt_red * ntiles_n;  // tiles per group
-    const int64_t c_all = red_cost_scan<BK, NS>(s_offs, groups, s_scan, &s_cmax) * (int64_t)tpg;
-    skew = (int64_t)s_cmax * 2 * gridDim.x > c_all;
-    if (skew) {
-      for (int g = tid; g < groups; g += Cfg::NT) {
-        const int c = s_scan[g + 1] - s_scan[g];
-        int r = 0;
-        for (int h = 0; h < groups; ++h) {
-          const int ch = s_scan[h + 1] - s_scan[h];
-          r += (ch > c || (ch == c && h < g)) ? 1 : 0;
-        }
-        s_order[r] = g;
-      }
-      __syncthreads();
-      for (int x = 0; x < xcd; ++x) spos += ((int)gridDim.x - x + 7) >> 3;
-      spos += bi;
-      // spos < 0 from here on: this block's tiles are the list in s_scan
-      if (deal_below_mean<Cfg::NT>(s_order, s_scan, groups, tpg, total, c_all, (int)gridDim.x, spos, smem, s_deal))
-        spos = -1;
-    } else {
-      const int b0 = red_cost_tile(s_scan, groups, tpg, c_all * xcd / 8);
-      const int b1 = xcd == 7 ? total : red_cost_tile(s_scan, groups, tpg, c_all * (xcd + 1) / 8);
-      start = b0;
-      cnt = b1 - b0;
-    }
-  } else {
-    const int per = total >> 3, rem = total & 7;
-    cnt = per + (xcd < rem ? 1 : 0);
-    start = xcd * per + (xcd < rem ? xcd : rem);
-  }
-  // The k-th tile of this block (k = 0, 1, ...) as a list index, or -1 past its last.
-  auto tile_at = [&](int k) -> int {
-    if (skew) {
-      if (spos < 0) {
-        const int j = k < kMaxDealt ? s_scan[k] : -1;  // this block's k-th tile in the cost order
-        return j < 0 ? -1 : s_order[j / tpg] * tpg + j % tpg;
-      }
-      const int NB = (int)gridDim.x;
-      const int j = k * NB + ((k & 1) ? NB - 1 - spos : spos);
-      return j < total ? s_order[j / tpg] * tpg + j % tpg : -1;
-    }
-    const int b = bi + k * nb;
-    return b < cnt ? start + b : -1;
-  };
-  if (tile_at(0) < 0) return;
+  const int ntiles_n = walk.ntiles_n, mt_red = walk.mt_red, mb = walk.mb;
+  auto tile_at = [&](int k) { return walk.at(k); };
 
   const uint32_t lds0 = lds_addr(smem);
   float* stage = s_epi + wave * SLAB * EpiStage<Cfg, PACK, SLAB>::ROW;
@@ -1128,17 +1161,13 @@ hipError_t expert_gemm_persist_rows(int kind, const T16* A, const T16* B, const 
   return hipErrorInvalidValue;
 }
 
-// The six expert GEMMs on the persistent kernel; Tw is the weight gradients'
-// type (the operands' 16-bit format, or fp32 for fp32 master weights: the
-// accumulators stored unrounded). A gathered operand takes the GATH instance
-// of its GEMM.
+// The weight gradients on the persistent kernel; Tw is their type (the
+// operands' 16-bit format, or fp32 for fp32 master weights: the accumulators
+// stored unrounded). A gathered operand takes the GATH instance of its GEMM.
 template <class Cfg, typename Tw = typename Cfg::Tc, typename T16 = typename Cfg::Tc>
-hipError_t expert_gemm_persist(int kind, const T16* A, const T16* B, const T16* aux, T16* C, T16* C2, Tw* Cw,
-                               const int32_t* offs, int P, int E, int H, int I, const ExpertGather& xg, int num_cus,
-                               hipStream_t s) {
-  if (kind != EG_DOWN_WGRAD && kind != EG_GATE_UP_WGRAD)
-    return expert_gemm_persist_rows<Cfg>(kind, A, B, aux, C, C2, offs, P, E, H, I, xg, num_cus, s);
-  GemmParams p = expert_params(kind, A, B, aux, C, C2, offs, P, E, H, I, xg);
+hipError_t expert_gemm_persist_wgrad(int kind, const T16* A, const T16* B, Tw* Cw, const int32_t* offs, int P, int E,
+                                     int H, int I, const ExpertGather& xg, int num_cus, hipStream_t s) {
+  GemmParams p = expert_params<T16>(kind, A, B, nullptr, nullptr, nullptr, offs, P, E, H, I, xg);
   p.C = Cw;
   if (xg.index == nullptr) return launch_gemm_persist<Cfg, false, false, GM_RED, EPI_STORE, Tw>(p, num_cus, s);
   if (kind == EG_DOWN_WGRAD) return launch_gemm_persist<Cfg, false, false, GM_RED, EPI_STORE, Tw, GA_KROWS>(p, num_cus, s);
