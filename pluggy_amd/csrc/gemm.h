@@ -662,19 +662,4 @@ GemmParams expert_params(int kind, const T* A, const T* B, const T* aux, T* C, T
   return p;
 }
 
-template <class Cfg, typename T>
-hipError_t expert_gemm(int kind, const T* A, const T* B, const T* aux, T* C, T* C2, const int32_t* offs, int P,
-                       int E, int H, int I, const ExpertGather& xg, hipStream_t s) {
-  const GemmParams p = expert_params<T>(kind, A, B, aux, C, C2, offs, P, E, H, I, xg);
-  switch (kind) {
-    case EG_GATE_UP_FWD: return launch_gemm<Cfg, T, T, T, true, true, GM_ROWS, EPI_SWIGLU>(p, s);
-    case EG_DOWN_FWD: return launch_gemm<Cfg, T, T, T, true, true, GM_ROWS, EPI_STORE>(p, s);
-    case EG_DOWN_DGRAD: return launch_gemm<Cfg, T, T, T, true, false, GM_ROWS, EPI_SWIGLU_BWD>(p, s);
-    case EG_DOWN_WGRAD: return launch_gemm<Cfg, T, T, T, false, false, GM_RED, EPI_STORE>(p, s);
-    case EG_GATE_UP_DGRAD: return launch_gemm<Cfg, T, T, T, true, false, GM_ROWS, EPI_STORE>(p, s);
-    case EG_GATE_UP_WGRAD: return launch_gemm<Cfg, T, T, T, false, false, GM_RED, EPI_STORE>(p, s);
-  }
-  return hipErrorInvalidValue;
-}
-
 }  // namespace pmoe

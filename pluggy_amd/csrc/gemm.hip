@@ -3,20 +3,16 @@
 
 #include "gemm_persist.h"
 #include "gemm_pingpong.h"
+#include "gemm_split.h"
 #include "kernels.h"
 
 namespace pmoe {
 
 namespace {
 
-// Tile shapes of the register-staged engine: fp32 (MFMA 32x32x2) uses 64x128
-// blocks of four 32x64 wave tiles.
-typedef TileCfg<bf16_t, 128, 128, 64, 64> CfgBf16;
+// Tile shape of the register-staged engine, which runs the fp32 router's GEMMs
+// (MFMA 32x32x2): 64x128 blocks of four 32x64 wave tiles.
 typedef TileCfg<float, 64, 128, 32, 64> CfgF32;
-
-template <typename T> struct CfgFor;
-template <> struct CfgFor<bf16_t> { typedef CfgBf16 type; };
-template <> struct CfgFor<float> { typedef CfgF32 type; };
 
 // The weight gradients run on the persistent DMA engine: 256x256 blocks of
 // eight 128x64 wave tiles (two waves per SIMD, one block per CU) with a
@@ -109,7 +105,7 @@ bool use_rows128(int kind, int P, int E, int H, int I, int cus) {
 }  // namespace
 
 int expert_gemm_tile_rows(int kind, int P, int E, int H, int I, bool half, int cus) {
-  if (!half) return CfgF32::BM;
+  if (!half) return SplitCfg::BM;
   if (cus <= 0) cus = num_cus();
   if ((kind == EG_GATE_UP_FWD || kind == EG_DOWN_FWD) && (int64_t)P <= (int64_t)kDecodeRowsPerExpert * E)
     return DmaDecode::BM;
@@ -134,7 +130,8 @@ hipError_t expert_gemm_run(int kind, const T* A, const T* B, const T* aux, T* C,
     return expert_gemm_persist_wgrad<typename Cfgs::Main, Tw>(kind, A, B, Cw, offs, P, E, H, I, xg, num_cus(), s);
   } else {
     static_assert(std::is_same<T, Tw>::value, "fp32 operands give fp32 weight gradients");
-    return expert_gemm<typename CfgFor<T>::type, T>(kind, A, B, aux, wgrad ? Cw : C, C2, offs, P, E, H, I, xg, s);
+    const GemmParams p = expert_params<T>(kind, A, B, aux, wgrad ? Cw : C, C2, offs, P, E, H, I, xg);
+    return expert_gemm_split(kind, p, s);
   }
 }
 

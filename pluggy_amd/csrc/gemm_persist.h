@@ -136,9 +136,9 @@ __device__ __forceinline__ void store_tile_full_cols(const f32x16 (&acc)[Cfg::MI
   const int r = lane / CPR, c = (lane % CPR) * 8;
   const int ld_bytes = (int)(p.ldc * sizeof(Tout));
   constexpr int AUX = NT ? 2 : 0;  // nt
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    if (i >= blocks) break;
+  static_for<0, MI>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    if (i >= blocks) return;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -157,7 +157,7 @@ __device__ __forceinline__ void store_tile_full_cols(const f32x16 (&acc)[Cfg::MI
         __builtin_amdgcn_raw_buffer_store_b128(hi, rs, off + 16, 0, AUX);
       }
     }
-  }
+  });
 }
 
 // Epilogue of the SwiGLU backward (down dgrad, EPI_SWIGLU_BWD) for a tile
@@ -299,9 +299,9 @@ __device__ __forceinline__ void store_slabs(const f32x16 (&acc)[Cfg::MI][Cfg::NI
           wsp[i][hs][ei] = (p.row_w != nullptr && e < SLAB * SW_CPR && row < ti.m_end) ? p.row_w[row] : 1.0f;
         }
   }
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    if (i >= blocks) break;
+  static_for<0, MI>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    if (i >= blocks) return;
 #pragma unroll
     for (int hs = 0; hs < NSL; ++hs) {
       if constexpr (PACK) {
@@ -360,7 +360,9 @@ __device__ __forceinline__ void store_slabs(const f32x16 (&acc)[Cfg::MI][Cfg::NI
         static_assert(EPI != EPI_SWIGLU_BWD || WN == 64, "routing-weight partials are per 64-column block");
         const int col_base = ti.n0 + wn * WN;
 #pragma unroll
-        for (int e = lane; e < SLAB * CPR; e += 64) {
+        for (int ei = 0; ei < (SLAB * CPR + 63) / 64; ++ei) {
+          const int e = lane + 64 * ei;
+          if (e >= SLAB * CPR) break;
           const int r = e / CPR, c = (e % CPR) * 8;
           const int row = row_base + r, col = col_base + c;
           float pd = 0.0f;  // this lane's share of <acc, silu(g) u> (EPI_SWIGLU_BWD with row_w)
@@ -415,7 +417,7 @@ __device__ __forceinline__ void store_slabs(const f32x16 (&acc)[Cfg::MI][Cfg::NI
       }
       // (the next slab's writes follow these reads in the wave's LDS order)
     }
-  }
+  });
 }
 
 // Of D DMAs placed after MFMA slots (i * TOTM) / D, those before slot PRE.

@@ -15,7 +15,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from tests._gpu_helpers import DEV, MAX_ABS_FRAC, check_close, gen, ref_grouped, say
+from tests._gpu_helpers import DEV, MAX_ABS_FRAC, check_close, gen, ref_grouped, ref_wgrad, say
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +63,60 @@ def test_row_grouped_tile_edges(rows, H, I, dtype):
     check_close("dw", part.sum(1, dtype=torch.float64), (dm * gate * s * up).sum(1), 1e-5, 1e-5)
     gx = ops.gate_up_dgrad(ggu, wgu.to(DEV), offs)
     check_close("dx_perm", gx, ref_grouped(ggu.cpu(), wgu, o, trans_w=False), tol, mx)
+
+
+def _f32_case(rows, H, I, seed):
+    from pluggy_amd import ops
+
+    E, P = len(rows), sum(rows)
+    g = gen(seed)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(P, generator=g)].reshape(-1, 1)
+    x = torch.randn(P, H, generator=g)
+    w = torch.rand(P, 1, generator=g) + 0.5
+    wgu = torch.randn(E, 2 * I, H, generator=g) * 0.1
+    wdn = torch.randn(E, H, I, generator=g) * 0.1
+    _, offs, _, _, tok, sw = ops.permute_rows(ids.to(DEV), w.to(DEV), E)
+    return ops, x, wgu, wdn, offs, tok, sw
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-25, 1e25])
+@pytest.mark.parametrize("H, I", [(40, 24), (512, 264)])
+def test_fp32_gemms_are_fp32_exact(H, I, scale):
+    """fp32 operands through their bf16 pieces: the error against fp64 is that of
+    fp32 sums. A sum of n products accumulated in fp32 in any order is off by at
+    most n 2^-24 of the sum of magnitudes; roundings of random sign give about
+    sqrt(n) 2^-24 of the result's norm, allowed twice (the pieces left out, 2^-23
+    of a product at worst, are inside that)."""
+    ops, x, wgu, wdn, offs, tok, sw = _f32_case([64, 65, 1, 0, 200, 63], H, I, 5)
+    x = x * scale
+    say(f"fp32 GEMMs H={H} I={I} scale={scale}")
+    bound = lambda n: 2.0 * max(n, 4) ** 0.5 * 2.0 ** -24  # noqa: E731
+    o, t = offs.cpu(), tok.cpu().long()
+    gu, _ = ops.gate_up_swiglu(x.to(DEV), wgu.to(DEV), offs, tok, sw)
+    check_close("gate_up", gu, ref_grouped(x[t], wgu, o, trans_w=True), bound(H), 1e-5)
+    a = x[:, :1].expand(-1, I).contiguous() * torch.linspace(0.5, 2.0, I)
+    y = ops.down_proj(a.to(DEV), wdn.to(DEV), offs)
+    check_close("y", y, ref_grouped(a, wdn, o, trans_w=True), bound(I), 1e-5)
+    gg = torch.cat([a, -a], dim=1)
+    gx = ops.gate_up_dgrad(gg.to(DEV), wgu.to(DEV), offs)
+    check_close("dx_perm", gx, ref_grouped(gg, wgu, o, trans_w=False), bound(2 * I), 1e-5)
+    gw = ops.gate_up_wgrad(gg.to(DEV), wgu[0, :1].expand(x.shape[0], -1).contiguous().to(DEV), offs, len(wgu))
+    check_close("dgate_up", gw, ref_wgrad(gg, wgu[0, :1].expand(x.shape[0], -1).contiguous(), o), bound(200), 1e-5)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), -float("inf"), float("nan")])
+def test_fp32_gemms_keep_infinities(bad):
+    """A row with an infinity or NaN gives the infinities and NaNs of fp32
+    arithmetic, and the other rows of its tile their values."""
+    H, I = 64, 40
+    ops, x, wgu, wdn, offs, tok, sw = _f32_case([70, 30], H, I, 9)
+    say(f"fp32 GEMMs with {bad}")
+    x[17, 5] = bad
+    t = tok.cpu().long()
+    gu, _ = ops.gate_up_swiglu(x.to(DEV), wgu.to(DEV), offs, tok, sw)
+    ref = ref_grouped(x[t], wgu, offs.cpu(), trans_w=True)
+    got, fine = gu.cpu().double(), torch.isfinite(ref)
+    assert torch.equal(fine, torch.isfinite(got)) and torch.equal(torch.isnan(ref), torch.isnan(got))
+    assert torch.equal(ref[~fine].nan_to_num(nan=0.0), got[~fine].nan_to_num(nan=0.0))
+    assert int((~fine).any(dim=1).sum()) == 1
+    check_close("finite rows", got[fine], ref[fine], 1e-6, 1e-5)
