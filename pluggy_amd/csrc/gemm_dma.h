@@ -123,6 +123,42 @@ __device__ __forceinline__ void dma16(const BufRsrc& rs, uint32_t lds, uint32_t 
         : "memory");
 }
 
+// Two of them, the second STEP bytes on in LDS.
+template <int STEP, bool NTL = false>
+__device__ __forceinline__ void dma16x2(const BufRsrc& rs, uint32_t lds, uint32_t voff0, uint32_t voff1) {
+  uint32_t m;
+  if constexpr (NTL)
+    asm volatile(
+        "s_nop 4\n\t"
+        "buffer_load_dwordx4 %1, %3, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, %5\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %3, 0 offen nt lds"
+        : "={m0}"(m)
+        : "v"(voff0), "v"(voff1), "s"(rs), "0"(lds), "n"(STEP)
+        : "memory", "scc");
+  else
+    asm volatile(
+        "s_nop 4\n\t"
+        "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, %5\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %3, 0 offen lds"
+        : "={m0}"(m)
+        : "v"(voff0), "v"(voff1), "s"(rs), "0"(lds), "n"(STEP)
+        : "memory", "scc");
+}
+
+// The same for 4 bytes per lane (lane l's dword goes to lds + 4*l).
+__device__ __forceinline__ void dma4(const BufRsrc& rs, uint32_t lds, uint32_t voff) {
+  asm volatile(
+      "s_nop 4\n\t"
+      "buffer_load_dword %0, %1, 0 offen lds"
+      :
+      : "v"(voff), "s"(rs), "{m0}"(lds)
+      : "memory");
+}
+
 // Block barrier for the DMA pipeline: waits for this wave's LDS reads only
 // (lgkmcnt(0)), never for outstanding DMA; fences compiler reordering.
 __device__ __forceinline__ void lds_barrier() {

@@ -22,6 +22,13 @@
 //    1 A0, 2 N1, 3 A1, all for two k tiles ahead, so a unit is fetched seven
 //    phases before it is read and 96-112 KiB are in flight, as in a ring of
 //    four 32-deep stages, but in 128-byte pieces.
+//
+// What bounds it (shader clocks of a block at 8192 tokens of the Qwen3-30B-A3B
+// layer): a k tile's MFMAs take 2048 clocks per SIMD; without its DMAs it runs
+// in 2115, with them in 2400-2550, the segments that read fragments and issue
+// DMAs being the longer ones: hence the checks kept out of them and the offsets
+// formed from one register per operand. At large sizes the chip's power is the
+// limit (the same launch on zero operands takes 397 us instead of 614).
 #pragma once
 
 #include "gemm_persist.h"
@@ -36,12 +43,6 @@ struct PpCfg : DmaCfg<256, 256, 128, 64, 2, 64, 1, Tc_> {
   static constexpr int ROW_SPAN = 192;
   __device__ static constexpr int wave_row(int wm) { return wm * 64; }
   __device__ static constexpr int row_blk(int i) { return (i >> 1) * 128 + (i & 1) * 32; }
-};
-
-// One DMA'd 16 KiB unit: two 1 KiB instructions per wave. off: this lane's
-// byte offset at the unit's first k, or kOOB.
-struct PpUnit {
-  uint32_t off[2];
 };
 
 template <class Cfg, typename Tout, bool B_KC, int EPI, int GATH>
@@ -62,6 +63,8 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
   __shared__ __attribute__((aligned(16))) float s_epi[EpiStage<Cfg, PACK, SLAB>::WORDS];
   __shared__ int s_scan[1025];
   __shared__ int s_offs[1024];
+  __shared__ __attribute__((aligned(16))) int s_tile[64][4];  // group, m0, m_end, n0 of the block's tiles, a ring
+  __shared__ int s_idx[GATH == GA_ROWS ? 2 : 1][GATH == GA_ROWS ? 256 : 1];  // row indices of two tiles
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -73,7 +76,6 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
   if (!walk.init(p, (EPI == EPI_SWIGLU) ? p.inter : p.N, (EPI == EPI_SWIGLU) ? BN / 2 : BN, s_offs, s_scan, nullptr,
                  nullptr, nullptr, nullptr))
     return;
-  const int ntiles_n = walk.ntiles_n, mb = walk.mb;
 
   const uint32_t lds0 = lds_addr(smem);
   float* stage = s_epi + wave * SLAB * EpiStage<Cfg, PACK, SLAB>::ROW;
@@ -91,121 +93,136 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
     asm volatile("" : "+v"(l));
     return l;
   };
-  const uint32_t ldb2 = (uint32_t)(p.ldb * 2);
+  const uint32_t lda2 = (uint32_t)(p.lda * 2), ldb2 = (uint32_t)(p.ldb * 2);
 
-  // A tile: its place and descriptors (wave-uniform), and this lane's DMA offsets.
+  // Where the block's tiles lie is worked out for many at once (a lane each, in
+  // a ring of 64 entries refilled by halves), and the rows a gathered tile
+  // reads are fetched to LDS two tiles ahead: a tile's set-up is then one LDS
+  // read and a few multiplications, done in the k loop when the DMAs turn to
+  // it. (Searching the group and reading the indices through the scalar cache
+  // between the tiles took 2.3 K clocks a tile, 4.9 K with a gather; a tile's k
+  // loop takes 30 to 80 K.)
+  auto fill_tiles = [&](int first, int n) {
+    if (tid < n) {
+      const int t = walk.at(first + tid);
+      int e[4] = {-1, 0, 0, 0};
+      if (t >= 0) {
+        const int g = rows_group(s_scan, groups, t / walk.ntiles_n);
+        int mt, tn;
+        rows_tile(t - s_scan[g] * walk.ntiles_n, s_scan[g + 1] - s_scan[g], walk.ntiles_n, walk.mb, tn, mt);
+        e[0] = g;
+        e[1] = (g == 0 ? 0 : s_offs[g - 1]) + mt * BM;
+        e[2] = s_offs[g];
+        e[3] = tn * (EPI == EPI_SWIGLU ? BN / 2 : BN);
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x) s_tile[(first + tid) & 63][x] = e[x];
+    }
+    lds_barrier();
+  };
+  auto tile_info = [&](int k) {
+    TileInfo ti;
+    const int* e = s_tile[k & 63];
+    ti.group = __builtin_amdgcn_readfirstlane(e[0]);
+    ti.m0 = __builtin_amdgcn_readfirstlane(e[1]);
+    ti.m_end = __builtin_amdgcn_readfirstlane(e[2]);
+    ti.n0 = __builtin_amdgcn_readfirstlane(e[3]);
+    ti.k_lo = 0;
+    ti.k_hi = p.K;
+    return ti;
+  };
+  // Row indices of tile k (256 of them, 64 per wave; past the table's end: 0)
+  auto fetch_rows = [&](int k) {
+    if constexpr (GATH == GA_ROWS) {
+      if (wave < 4) {
+        const int m0 = __builtin_amdgcn_readfirstlane(s_tile[k & 63][1]);
+        const BufRsrc rs = make_rsrc(p.a_index + m0, (uint64_t)(p.n_index - m0) * 4);
+        dma4(rs, lds_addr(reinterpret_cast<const char*>(&s_idx[k & 1][wave * 64])), (uint32_t)(wave * 64 + lane) * 4);
+      }
+    }
+  };
+
+  // What the DMAs fetch: a tile's place, its descriptors (wave-uniform) and this
+  // lane's offsets.
   struct LoadTile {
     TileInfo ti;
     BufRsrc rsA, rsB;
+    // Byte offsets of this lane's chunks (kOOB: none). The four of an operand's
+    // k tile (two units of two instructions) lie at fixed distances, except
+    // for gathered rows and SwiGLU columns (which end inside B, not at its end).
+    uint32_t a[GATH == GA_ROWS ? 4 : 1], b[EPI == EPI_SWIGLU ? 2 : 1];
+    bool half;  // at most 128 rows: A1 is neither fetched nor read
+    // a half tile that is its group's only m-tile: no other tile reads its B, which
+    // streams in with non-temporal loads (1200 tokens of the Qwen3-30B-A3B layer:
+    // the four GEMMs 592 -> 542 us)
+    bool stream;
   };
-  struct Offsets {
-    PpUnit a[2];
-    PpUnit b[B_KC ? 2 : 1];  // [k][n]: both halves share their offsets (32 k-rows apart)
-  };
-  constexpr int NOFF = sizeof(Offsets) / 4;
-  auto setup = [&](int t, LoadTile& T, Offsets& O) {
-    const int l = fresh_lane();
-    const int kc_row = l >> 3;
-    T.ti.group = 0; T.ti.m0 = 0; T.ti.m_end = 0; T.ti.n0 = 0; T.ti.k_lo = 0; T.ti.k_hi = 0;
-    const bf16_t* a_base = A0;
-    const bf16_t* b_base = B0;
-    uint64_t a_bytes = 0, b_bytes = 0;
-    if (t >= 0) {
-      const int g = rows_group(s_scan, groups, t / ntiles_n);
-      const int lo = g == 0 ? 0 : s_offs[g - 1];
-      int tn, mt;
-      rows_tile(t - s_scan[g] * ntiles_n, s_scan[g + 1] - s_scan[g], ntiles_n, mb, tn, mt);
-      T.ti.group = g; T.ti.m0 = lo + mt * BM; T.ti.m_end = s_offs[g];
-      T.ti.n0 = (EPI == EPI_SWIGLU) ? tn * (BN / 2) : tn * BN;
-      T.ti.k_hi = p.K;
-      b_base = B0 + (int64_t)g * p.strideB;
-      b_bytes = p.b_bytes;
-      if constexpr (GATH == GA_ROWS) {
-        a_bytes = p.a_bytes;  // the whole gathered storage
-      } else {
-        a_base = A0 + (int64_t)T.ti.m0 * p.lda;
-        a_bytes = (uint64_t)(T.ti.m_end - T.ti.m0) * p.lda * 2;
-      }
-    }
-    T.rsA = make_rsrc(a_base, a_bytes);
-    T.rsB = make_rsrc(b_base, b_bytes);
+  auto load_tile = [&](int k, LoadTile& T) {
+    const int l = fresh_lane(), kc_row = l >> 3;
+    T.ti = tile_info(k);
     const int rows = T.ti.m_end - T.ti.m0;
-    // A halves: LDS row r of half h is tile row 128 h + r
+    T.half = rows <= BM / 2;
+    T.stream = T.half && T.ti.m0 == (T.ti.group > 0 ? __builtin_amdgcn_readfirstlane(s_offs[max(T.ti.group, 1) - 1]) : 0);
+    const bool any = T.ti.group >= 0;  // past the block's last tile every DMA reads zeros
+    const int g = any ? T.ti.group : 0;
+    if constexpr (GATH == GA_ROWS) T.rsA = make_rsrc(A0, any ? p.a_bytes : 0);  // the whole gathered storage
+    else T.rsA = make_rsrc(A0 + (int64_t)T.ti.m0 * p.lda, (uint64_t)rows * lda2);
+    T.rsB = make_rsrc(B0 + (int64_t)g * p.strideB, any ? p.b_bytes : 0);
+    // A halves: LDS row r of half h is tile row 128 h + r; rows past the group's
+    // end lie past the descriptor's bound
+    const int r0 = 8 * wave + kc_row;
+    if constexpr (GATH == GA_ROWS) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+      for (int x = 0; x < 4; ++x)
+        T.a[x] = r0 + 64 * x < rows ? (uint32_t)s_idx[k & 1][r0 + 64 * x] * lda2 + (uint32_t)(kc_k * 2) : kOOB;
+    } else {
+      T.a[0] = (uint32_t)r0 * lda2 + (uint32_t)(kc_k * 2);
+    }
+    if constexpr (EPI == EPI_SWIGLU) {
+      // N halves: half 0 holds gate columns (LDS row r: tile column r), half 1 the matching up columns
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const int rb = 128 * h + 8 * (wave + i * NW);
-        const int r = rb + kc_row;
-        int64_t src = r;
-        if constexpr (GATH == GA_ROWS) {
-          // 8 consecutive rows per instruction: their indices come through the
-          // scalar cache (uniform addresses, clamped into the table)
-          typedef const __attribute__((address_space(4))) int32_t cint;
-          cint* ci = (cint*)p.a_index;
-          const int64_t last = p.n_index - 1;
-          const int m0 = __builtin_amdgcn_readfirstlane(T.ti.m0);
-          int tok = 0;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int v = ci[min<int64_t>((int64_t)m0 + rb + j, last)];
-            tok = kc_row == j ? v : tok;
-          }
-          src = tok;
-        }
-        O.a[h].off[i] = r < rows ? (uint32_t)((src * p.lda + kc_k) * 2) : kOOB;
+        const int col = T.ti.n0 + r0 + 64 * i;
+        T.b[i] = col < p.inter ? (uint32_t)col * ldb2 + (uint32_t)(kc_k * 2) : kOOB;
       }
-    if constexpr (B_KC) {
-      // N halves: LDS row r of half n is tile column 64 (r / 32) + 32 n + r % 32;
-      // with SwiGLU half 0 holds gate columns and half 1 the matching up columns
-#pragma unroll
-      for (int n = 0; n < 2; ++n)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int r = 8 * (wave + i * NW) + kc_row;
-          int col;
-          bool ok;
-          if constexpr (EPI == EPI_SWIGLU) {
-            col = T.ti.n0 + r;  // 32 columns per wave
-            ok = col < p.inter;
-            col += n * p.inter;
-          } else {
-            col = T.ti.n0 + 64 * (r >> 5) + 32 * n + (r & 31);
-            ok = col < p.N;
-          }
-          O.b[n].off[i] = ok ? (uint32_t)(((int64_t)col * p.ldb + kc_k) * 2) : kOOB;
-        }
+    } else if constexpr (B_KC) {
+      // LDS row r of half n is tile column 64 (r / 32) + 32 n + r % 32 (the end of B is the descriptor's)
+      T.b[0] = (uint32_t)(T.ti.n0 + 64 * (r0 >> 5) + (r0 & 31)) * ldb2 + (uint32_t)(kc_k * 2);
     } else {
       // [k][n] unit: 32 k-rows of 256 columns, 2 k-rows per instruction
       const int t_kk = 2 * wave + (l >> 5);
       const int col = T.ti.n0 + 8 * ((l & 31) ^ swz_t(t_kk));
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        O.b[0].off[i] = col < p.N ? (uint32_t)(t_kk + 2 * i * NW) * ldb2 + (uint32_t)(col * 2) : kOOB;
+      T.b[0] = col < p.N ? (uint32_t)t_kk * ldb2 + (uint32_t)(col * 2) : kOOB;
     }
   };
 
   // Unit U of k tile kt of T (0: N0, 1: A0, 2: N1, 3: A1) into the slot of parity par.
-  auto dma_unit = [&](const LoadTile& T, const Offsets& O, auto uc, int kt, int par) {
+  // WHOLE: of a whole k tile, and A1 too (nothing to check).
+  auto dma_unit = [&](const LoadTile& T, auto uc, auto whole, int kt, int par) {
     constexpr int U = decltype(uc)::value;
-    constexpr bool IS_A = U & 1;
+    constexpr bool IS_A = U & 1, WHOLE = decltype(whole)::value;
     constexpr int HALF = U >> 1;
+    if (!WHOLE && U == 3 && T.half) return;
     const uint32_t dst = lds0 + (IS_A ? 0 : 4 * UNIT) + (uint32_t)par * (2 * UNIT) + HALF * UNIT + wave * 1024;
     const int k0 = kt * BK;
+    uint32_t v[2];
     if constexpr (IS_A || B_KC) {
-      const PpUnit& u = IS_A ? O.a[HALF] : O.b[B_KC ? HALF : 0];
-      uint32_t v[2] = {u.off[0] + (uint32_t)(k0 * 2), u.off[1] + (uint32_t)(k0 * 2)};
-      const bool out = k0 + BK > p.K && k0 + kc_k >= p.K;  // the k tail
-      v[0] = out ? kOOB : v[0];
-      v[1] = out ? kOOB : v[1];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) dma16(IS_A ? T.rsA : T.rsB, dst + i * NW * 1024, v[i]);
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t k2 = (uint32_t)(k0 * 2);
+        if constexpr (IS_A && GATH == GA_ROWS) v[i] = T.a[2 * HALF + i] + k2;
+        else if constexpr (IS_A) v[i] = T.a[0] + (k2 + (uint32_t)(128 * HALF + 64 * i) * lda2);
+        else if constexpr (EPI == EPI_SWIGLU) v[i] = T.b[i] + (k2 + (HALF ? (uint32_t)p.inter * ldb2 : 0u));
+        else v[i] = T.b[0] + (k2 + (uint32_t)(32 * HALF + 128 * i) * ldb2);
+        if constexpr (!WHOLE) v[i] = k0 + BK > p.K && k0 + kc_k >= p.K ? kOOB : v[i];  // the k tail
+      }
     } else {
       // k-rows past K lie past the descriptor's bound and read as zero
-      const uint32_t base = (uint32_t)(k0 + 32 * HALF) * ldb2;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) dma16(T.rsB, dst + i * NW * 1024, __builtin_elementwise_add_sat(O.b[0].off[i], base));
+      for (int i = 0; i < 2; ++i) v[i] = __builtin_elementwise_add_sat(T.b[0], (uint32_t)(k0 + 32 * HALF + 16 * i) * ldb2);
     }
+    if (!WHOLE && !IS_A && T.stream) dma16x2<NW * 1024, true>(T.rsB, dst, v[0], v[1]);
+    else dma16x2<NW * 1024>(IS_A ? T.rsA : T.rsB, dst, v[0], v[1]);
   };
 
   // Lane addresses of the fragments within the operand's LDS region (parity
@@ -248,7 +265,7 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
   };
 
   f32x16 acc[MI][NI];
-  auto mfmas = [&](auto pc) {
+  auto mfmas = [&](auto pc) {  // of phase P
     constexpr int P = decltype(pc)::value, h = P >> 1, n = P & 1;
     __builtin_amdgcn_s_setprio(1);
     if constexpr (B_KC) {
@@ -277,34 +294,27 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // The next tile's offsets wait in the wave's part of the epilogue's LDS, free
-  // while k tiles run: only one set is held in registers.
-  static_assert(NOFF * 64 <= SLAB * EpiStage<Cfg, PACK, SLAB>::ROW, "a tile's offsets fit the wave's staging");
-  uint32_t* st_off = reinterpret_cast<uint32_t*>(stage) + lane;
-  LoadTile cur, nxt, ld;
-  Offsets off;
-  auto park = [&](const Offsets& O) {
-    const uint32_t* o = &O.a[0].off[0];
-#pragma unroll
-    for (int x = 0; x < NOFF; ++x) st_off[x * 64] = o[x];
-  };
   const int nk = max((p.K + BK - 1) / BK, 2);  // k tiles of every output tile
-  int tile = 0;
-  {
-    Offsets o;
-    setup(walk.at(1), nxt, o);
-    park(o);
-  }
-  setup(walk.at(0), cur, off);
-  ld = cur;
+  constexpr auto kAny = std::integral_constant<bool, false>();
+  constexpr auto kWhole = std::integral_constant<bool, true>();
+  LoadTile ld;
+  fill_tiles(0, 64);
+  fetch_rows(0);
+  fetch_rows(1);
+  wait_vmcnt<0>();
+  lds_barrier();
+  load_tile(0, ld);
+  TileInfo cur = ld.ti;
+  bool half = ld.half;
 #pragma unroll
   for (int kt = 0; kt < 2; ++kt)
-    static_for<0, 4>([&](auto uc) { dma_unit(ld, off, uc, kt, kt); });
+    static_for<0, 4>([&](auto uc) { dma_unit(ld, uc, kAny, kt, kt); });
   wait_vmcnt<0>();
   lds_barrier();
   read_n(std::integral_constant<int, 0>());
   lds_barrier();  // N0's slot is refilled in phase 0
-  int par = 0;
+  int par = 0, tile = 0;
+  const int lean_end = (p.K & (BK - 1)) == 0 ? nk - 2 : nk - 3;  // k tiles whose DMAs fetch whole k tiles of this tile
 
   for (;;) {
 #pragma unroll
@@ -313,17 +323,25 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
       for (int j = 0; j < NI; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    // A row-grouped tile of at most 128 rows needs A0 alone: two phases a k tile.
-    const bool half = cur.ti.m_end - cur.ti.m0 <= BM / 2;
+    if (((tile + 2) & 31) == 0) fill_tiles(tile + 2, 32);
+    // A tile's indices landed before the previous epilogue in the waves that fetched
+    // them; with two k tiles no phase's barrier lies between that and their use.
+    if (GATH == GA_ROWS && nk == 2) lds_barrier();
+    fetch_rows(tile + 2);
     if (second) swap_groups();
-    // Phase P of k tile kt, whose DMAs fetch unit P of k tile lkt of T (two k
-    // tiles on). Ahead of a phase's end lie the units of the next six phases,
-    // two instructions each, so a wait for vmcnt(12) leaves the next phase's
-    // unit landed. A tile's first seven units landed before its first phase
+    // Phase P of k tile kt, whose DMAs fetch unit P of k tile lkt (two k tiles
+    // on). Ahead of a phase's end lie the units of the next six phases, two
+    // instructions each, so a wait for vmcnt(12) leaves the next phase's unit
+    // landed (8: two of the six may be A1s not fetched for a next tile that is
+    // a half one). A tile's first seven units landed before its first phase
     // (the prologue, or the wait before the epilogue): no wait until phase 6,
     // which gives the epilogue's stores, counted with the loads, six phases.
-    auto phase = [&](auto pc, int kt, int lkt) {
+    // The phases between the first two and the last k tiles (`lean`) check
+    // none of that: their reads and DMAs are what a segment's length hangs on
+    // (the checks there cost 6 to 10 % of the GEMMs' time).
+    auto phase = [&](auto pc, auto lean, int kt, int lkt, bool few) {
       constexpr int P = decltype(pc)::value;
+      constexpr bool LEAN = decltype(lean)::value;
       if constexpr (P == 3) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) lb[ks] ^= 2 * UNIT;
@@ -332,27 +350,33 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
       else if constexpr (P == 1) read_n(std::integral_constant<int, 1>());
       else if constexpr (P == 2) read_a(std::integral_constant<int, 1>());
       else read_n(std::integral_constant<int, 0>());
-      dma_unit(ld, off, pc, lkt, par);
-      if (kt > 1 || (P >= 2 && kt == 1)) wait_vmcnt<12>();
+      dma_unit(ld, pc, lean, lkt, par);
+      if constexpr (LEAN) {
+        wait_vmcnt<12>();
+      } else if (kt > 1 || (P >= 2 && kt == 1)) {
+        if (few) wait_vmcnt<8>();
+        else wait_vmcnt<12>();
+      }
       __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0)
       swap_groups();
       mfmas(pc);
       swap_groups();
     };
-    auto k_tile = [&](int kt, int lkt) {
-      static_for<0, 4>([&](auto pc) { phase(pc, kt, lkt); });
+    auto k_tile = [&](auto lean, int kt, int lkt, bool few) {
+      static_for<0, 4>([&](auto pc) { phase(pc, lean, kt, lkt, few); });
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) la[ks] ^= 2 * UNIT;
       par ^= 1;
     };
-    // The half tile's k tile: its two phases read A0 and N1, then the next N0,
-    // and issue the four units in the same order (A1's rows read zero), so that
-    // tiles of both kinds follow each other.
+    // A tile of at most 128 rows: two phases a k tile. The first reads A0 and N1,
+    // the second the next N0, and they issue the units in the same order
+    // (without its own A1s), so that tiles of both kinds follow each other.
+    // Three units at least follow the one each wait is for.
     auto half_k_tile = [&](int kt, int lkt) {
       read_a(std::integral_constant<int, 0>());
       read_n(std::integral_constant<int, 1>());
-      dma_unit(ld, off, std::integral_constant<int, 0>(), lkt, par);
-      if (kt > 0) wait_vmcnt<8>();  // the next k tile's N0
+      dma_unit(ld, std::integral_constant<int, 0>(), kAny, lkt, par);
+      if (kt > 0) wait_vmcnt<6>();  // the next k tile's N0
       __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));
       swap_groups();
       mfmas(std::integral_constant<int, 0>());
@@ -360,8 +384,8 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) lb[ks] ^= 2 * UNIT;
       read_n(std::integral_constant<int, 0>());
-      static_for<1, 4>([&](auto uc) { dma_unit(ld, off, uc, lkt, par); });
-      if (kt > 0) wait_vmcnt<10>();  // its A0 and N1
+      static_for<1, 4>([&](auto uc) { dma_unit(ld, uc, kAny, lkt, par); });
+      if (kt > 0) wait_vmcnt<6>();  // its A0 and N1
       __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));
       swap_groups();
       mfmas(std::integral_constant<int, 1>());
@@ -371,34 +395,31 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
       par ^= 1;
     };
     // From k tile nk - 2 on the DMAs fetch the next tile's first two.
-    auto to_next = [&]() {
-      ld = nxt;
-      uint32_t* o = &off.a[0].off[0];
-#pragma unroll
-      for (int x = 0; x < NOFF; ++x) o[x] = st_off[x * 64];
-    };
     if (half) {
 #pragma unroll 1
       for (int kt = 0; kt < nk; ++kt) {
-        if (kt == nk - 2) to_next();
-        half_k_tile(kt, kt < nk - 2 ? kt + 2 : kt + 2 - nk);
+        if (kt == nk - 2) load_tile(tile + 1, ld);
+        half_k_tile(kt, kt >= nk - 2 ? kt + 2 - nk : kt + 2);
       }
     } else {
 #pragma unroll 1
       for (int kt = 0; kt < nk; ++kt) {
-        if (kt == nk - 2) to_next();
-        k_tile(kt, kt < nk - 2 ? kt + 2 : kt + 2 - nk);
+        if (kt == 2) {
+#pragma unroll 1
+          for (; kt < lean_end; ++kt) k_tile(kWhole, kt, kt + 2, false);
+        }
+        const bool next = kt >= nk - 2;
+        if (kt == nk - 2) load_tile(tile + 1, ld);
+        k_tile(kAny, kt, next ? kt + 2 - nk : kt + 2, next && ld.half);
       }
     }
     if (!second) swap_groups();  // both groups store together
     wait_vmcnt<0>();             // the next tile's first two k tiles, before the stores join the count
-    store_slabs<Cfg, Tout, GM_ROWS, EPI, PACK, SLAB>(acc, stage, cur.ti, p, wm, wn, fresh_lane(), half ? MI / 2 : MI);
+    store_slabs<Cfg, Tout, GM_ROWS, EPI, PACK, SLAB>(acc, stage, cur, p, wm, wn, fresh_lane(), half ? MI / 2 : MI);
     ++tile;
-    if (walk.at(tile) < 0) break;
-    cur = nxt;
-    Offsets o;
-    setup(walk.at(tile + 1), nxt, o);
-    park(o);  // (after the epilogue's reads, in the wave's LDS order)
+    cur = ld.ti;
+    half = ld.half;
+    if (cur.group < 0) break;
   }
   wait_vmcnt<0>();  // the zero-reading DMAs past the last tile
 }
