@@ -113,8 +113,17 @@ struct SplitKc {  // k-contiguous: 8 chunks of 4 k per row
 };
 
 template <int R>
-struct SplitT {  // [k][r]: 4 k-rows x 4 columns per unit, 8 consecutive lanes on 8 k-blocks of one column block
+struct SplitT {  // [k][r]: 4 k-rows x 4 columns per unit
   static constexpr int UNITS = 8 * R / 4, PER_T = (UNITS + 255) / 256;
+  // Unit u's k-block and first column. Four consecutive lanes read 64 consecutive
+  // bytes of a k-row, and the 32 lanes of a half wave (four column blocks, 16 banks
+  // apart, by eight k-blocks of two banks) write all 64 LDS banks once. The six
+  // GEMMs with their moves, H 1024, E 32, I 512, top-4: with eight lanes on the
+  // k-blocks of one column block (a load touches a row per lane) 917 us at 2048
+  // tokens and 468 at 431, so 882 and 407; with eight lanes along a row (loads as
+  // good, LDS writes two to a bank) 913 and 469.
+  __device__ __forceinline__ static int k_of(int u) { return (u >> 2) & 7; }
+  __device__ __forceinline__ static int col_of(int u) { return ((u >> 5) * 4 + (u & 3)) * 4; }
   const float* base;
   int64_t ld;
   int r0, r_hi;
@@ -126,10 +135,10 @@ struct SplitT {  // [k][r]: 4 k-rows x 4 columns per unit, 8 consecutive lanes o
   __device__ __forceinline__ void load(int k0, int k_hi, int tid) {
 #pragma unroll
     for (int i = 0; i < PER_T; ++i) {
-      const int u = tid + i * 256, r = r0 + (u >> 3) * 4;
+      const int u = tid + i * 256, r = r0 + col_of(u);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int k = k0 + (u & 7) * 4 + j;
+        const int k = k0 + k_of(u) * 4 + j;
         u32x4 v = {0u, 0u, 0u, 0u};
         if ((UNITS % 256 == 0 || u < UNITS) && k < k_hi && r < r_hi)  // (r_hi is a multiple of 8: whole chunks)
           v = *reinterpret_cast<const u32x4*>(base + (int64_t)(kidx != nullptr ? kidx[k] : k) * ld + r);
@@ -148,7 +157,7 @@ struct SplitT {  // [k][r]: 4 k-rows x 4 columns per unit, 8 consecutive lanes o
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const u32x4 v = row(i, c);
-          Split4(v).put(lds + ((u >> 3) * 4 + c) * SplitCfg::ROW + (u & 7) * 8);
+          Split4(v).put(lds + (col_of(u) + c) * SplitCfg::ROW + k_of(u) * 8);
           m = max_abs4(v, m);
         }
       }
@@ -162,7 +171,7 @@ struct SplitT {  // [k][r]: 4 k-rows x 4 columns per unit, 8 consecutive lanes o
       if (UNITS % 256 == 0 || u < UNITS) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-          *reinterpret_cast<u32x4*>(lds + ((u >> 3) * 4 + c) * SplitCfg::LDF + (u & 7) * 4) = row(i, c);
+          *reinterpret_cast<u32x4*>(lds + (col_of(u) + c) * SplitCfg::LDF + k_of(u) * 4) = row(i, c);
       }
     }
   }
