@@ -89,6 +89,9 @@ int router_logit_splits(int64_t T, int64_t H, int64_t E, bool pieces) {
   s = std::min<int64_t>(s, std::min<int64_t>(kRouterMaxSplits, std::max<int64_t>(1, H / 256)));
   return (int)std::max<int64_t>(1, s);
 }
+// fp32 logits of at most this many experts come from the lane-split kernel
+// (router_logits_few), of more from the row-tile GEMM.
+constexpr int kRouterFewExperts = 32;
 int64_t router_splits(int64_t T) { return std::max<int64_t>(1, (T + kRouterSplitChunk - 1) / kRouterSplitChunk); }
 int64_t ldl_of(int64_t E) { return (E + 7) / 8 * 8; }
 
@@ -194,10 +197,12 @@ PMOE_API int pmoe_router_forward(const void* x, int x_dtype, const void* weight,
       nsplit = splits;
       sstride = (int64_t)T * E;
     } else {
-      hipError_t st = w_dtype == PMOE_F32
-                          ? router_logits_gemm<float, float>((const float*)x, (const float*)weight, t, h, e, logits, s)
-                          : router_logits_gemm<float, bf16_t>((const float*)x, (const bf16_t*)weight, t, h, e, logits,
-                                                              s);
+      const bool few = e <= kRouterFewExperts && ((uintptr_t)x | (uintptr_t)weight) % 16 == 0;
+      hipError_t st = by_dtype(w_dtype, [&](auto wp) {
+        typedef PMOE_ELEM(wp) W;
+        if (few) return router_logits_few<W>((const float*)x, (const W*)weight, t, h, e, logits, s);
+        return router_logits_gemm<float, W>((const float*)x, (const W*)weight, t, h, e, logits, s);
+      });
       PMOE_TRY(st, "router logits GEMM");
     }
     hipError_t st = by_dtype16(tw_dtype, [&](auto wp) {

@@ -708,3 +708,31 @@ def test_moe_expert_ffn_rejects_out_of_range_ids(bad):
     idx[5, 1] = 3
     out = pluggy_amd.moe_expert_ffn(args[0], idx.to(DEV), *args[2:])
     assert torch.isfinite(out).all()
+
+
+def _few_logits(x, W, K, **kw):
+    """router_forward's outputs, checked: logits to twice the error of an fp32 sum
+    of H products with roundings of random sign (sqrt(H) 2^-24 of the norm), ids
+    and statistics against the oracle on those logits."""
+    T, H, E = x.shape[0], x.shape[1], W.shape[0]
+    out = _ops().router_forward(x.to(DEV), W.to(DEV), K, True, **kw)
+    logits, _, ti, tw32, counts, psum, lse2 = out
+    assert rel(logits, x.double() @ W.double().t()) < 2.0 * max(H, 4) ** 0.5 * 2.0 ** -24
+    lg = logits.cpu()
+    sel = O.select_topk(lg, K)
+    assert np.array_equal(to_np(ti), sel)
+    rc, rps, rl2 = O.router_stats(lg, torch.from_numpy(sel), E)
+    assert np.array_equal(to_np(counts), rc.astype(np.int32))
+    assert rel(psum, rps) < 1e-5
+    assert abs(lse2.item() - rl2.item()) <= 1e-5 * abs(rl2.item()) + 1e-6
+    return out
+
+
+@pytest.mark.parametrize("T,H,E", [(1, 8, 1), (2, 72, 8), (15, 512, 9), (17, 264, 16), (33, 64, 17), (47, 1032, 32),
+                                   (47, 1032, 33)])
+def test_router_fp32_few_experts(T, H, E):
+    """fp32 rows at the edges of the few-expert logits kernel: 16 tokens a block,
+    8, 16 and 32 experts, H that its lanes share unevenly, and the GEMM beyond."""
+    say(f"fp32 router T={T} H={H} E={E}")
+    g = gen(T + H)
+    _few_logits(torch.randn(T, H, generator=g), torch.randn(E, H, generator=g) * 0.1, min(E, 3))
