@@ -736,3 +736,22 @@ def test_router_fp32_few_experts(T, H, E):
     say(f"fp32 router T={T} H={H} E={E}")
     g = gen(T + H)
     _few_logits(torch.randn(T, H, generator=g), torch.randn(E, H, generator=g) * 0.1, min(E, 3))
+
+
+@pytest.mark.parametrize("T", [1, 2, 4, 5, 8, 9, 16, 17])
+@pytest.mark.parametrize("H,E", [(8, 4), (264, 60), (2048, 128), (2056, 256), (264, 264)])
+def test_router_few_tokens(T, H, E):
+    """bf16 rows at the edges of the few-token logits kernel and of the one-block
+    statistics (16 tokens, 256 experts); the weight's pieces and an unaligned
+    weight give its logits too."""
+    say(f"few-token router T={T} H={H} E={E}")
+    g = gen(T + H)
+    x = torch.randn(T, H, generator=g).bfloat16()
+    W = torch.randn(E, H, generator=g) * 0.1
+    a = _few_logits(x, W, 4)
+    b = _few_logits(x, W, 4, pieces=_ops().split_router_weight(W.to(DEV)))
+    assert all(torch.equal(u, v) for u, v in zip(a, b))
+    odd = torch.cat([torch.zeros(1), W.reshape(-1)]).to(DEV)[1:].view(E, H)
+    assert odd.is_contiguous() and odd.data_ptr() % 16 == 4
+    c = _ops().router_forward(x.to(DEV), odd, 4, True)
+    assert rel(c[0], a[0].cpu().double()) < 1e-6 * max(H, 4) ** 0.5
