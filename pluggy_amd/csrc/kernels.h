@@ -29,7 +29,7 @@ int expert_gemm_tile_rows(int kind, int P, int E, int H, int I, bool half, int c
 // ---- router GEMMs in fp32 arithmetic (gemm.hip). TX: x dtype, TW: router weight dtype.
 template <typename TX, typename TW>
 hipError_t router_logits_gemm(const TX* x, const TW* w, int T, int H, int E, float* logits, hipStream_t s);
-// The same from fp32 x for E <= 32: H a multiple of 4, x rows 16-byte and w rows 4-element aligned (route.hip).
+// The same from fp32 x for few experts: H a multiple of 4, x rows 16-byte and w rows 4-element aligned (route.hip).
 template <typename TW>
 hipError_t router_logits_few(const float* x, const TW* w, int T, int H, int E, float* logits, hipStream_t s);
 // dx = dl . W   (dl: (T, ldl) fp32, columns >= E are ignored)

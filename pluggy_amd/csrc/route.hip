@@ -247,19 +247,23 @@ __device__ __forceinline__ f32x4 load4(const bf16_t* p) {
                __uint_as_float(v.y & 0xffff0000u)};
 }
 
-// fp32 router logits x . W^T of few experts (E <= EM): sixteen lanes share two
-// tokens and split the reduction over H, each lane four consecutive k of every
-// 64, with an accumulator per (token, expert) that is summed over the lanes at
-// the end (H / 16 terms a lane, then a tree of 16: shorter sums than a
+// fp32 router logits x . W^T of few experts, eight per block: sixteen lanes share
+// two tokens and split the reduction over H, each lane four consecutive k of
+// every 64, with an accumulator per (token, expert) that is summed over the lanes
+// at the end (H / 16 terms a lane, then a tree of 16: shorter sums than a
 // reduction in order). The row-tile GEMM has T / 64 blocks of one column tile
 // here, most of whose columns do not exist, on a chain of H / 2 fp32 MFMAs each;
-// this one has four times as many blocks, reads x once and finds the weight (at
-// most 32 rows) in cache. Forward of the block at H 512, E 8: 8000 tokens 454 ->
-// 438 us, 2048 tokens 175 -> 156, 317 tokens 107 -> 104.
-template <int EM, typename TW>
+// this one has four times as many blocks and finds the weight in cache. It is
+// bound by its weight loads, so eight accumulators a token: with 16 and 32 of
+// them in one block the router took 68 and 131 us at 8192 tokens of H 1024,
+// where the GEMM's takes 56 (24 for 16 in two blocks). Forward of the block at
+// H 512, E 8: 8000 tokens 454 -> 438 us, 2048 tokens 173 -> 156, 317 tokens 107
+// -> 104.
+template <typename TW>
 __global__ __launch_bounds__(128) void router_logits_few_kernel(const float* __restrict__ x, const TW* __restrict__ w,
                                                                int T, int H, int E, float* __restrict__ logits) {
-  const int lane = threadIdx.x & 63, li = lane & 15;
+  constexpr int EM = 8;
+  const int li = threadIdx.x & 15, e0 = blockIdx.y * EM;
   const int t0 = (blockIdx.x * 8 + (threadIdx.x >> 4)) * 2;
   // rows and experts past the end are read as the last ones and not written
   const float* x0 = x + (int64_t)min(t0, T - 1) * H;
@@ -272,7 +276,7 @@ __global__ __launch_bounds__(128) void router_logits_few_kernel(const float* __r
     const f32x4 b = *reinterpret_cast<const f32x4*>(x1 + k);
 #pragma unroll
     for (int e = 0; e < EM; ++e) {
-      const f32x4 v = load4(w + (int64_t)min(e, E - 1) * H + k);
+      const f32x4 v = load4(w + (int64_t)min(e0 + e, E - 1) * H + k);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         acc[0][e] = fmaf(a[i], v[i], acc[0][e]);
@@ -285,7 +289,7 @@ __global__ __launch_bounds__(128) void router_logits_few_kernel(const float* __r
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const float v = row16_sum(acc[j][e]);
-      if (li == (e & 15) && e < E && t0 + j < T) logits[(int64_t)(t0 + j) * E + e] = v;
+      if (li == e && e0 + e < E && t0 + j < T) logits[(int64_t)(t0 + j) * E + e0 + e] = v;
     }
 }
 
@@ -1197,14 +1201,8 @@ hipError_t split_bf16x3(const float* w, int64_t n, int planes, bf16_t* out, hipS
 template <typename TW>
 hipError_t router_logits_few(const float* x, const TW* w, int T, int H, int E, float* logits, hipStream_t s) {
   if (T == 0) return hipSuccess;
-  const unsigned grid = blocks_for(T, 16);
-#define PMOE_LOGITS_FEW(EM) \
-  hipLaunchKernelGGL((router_logits_few_kernel<EM, TW>), dim3(grid), dim3(128), 0, s, x, w, T, H, E, logits)
-  if (E <= 8) PMOE_LOGITS_FEW(8);
-  else if (E <= 16) PMOE_LOGITS_FEW(16);
-  else if (E <= 32) PMOE_LOGITS_FEW(32);
-  else return hipErrorInvalidValue;
-#undef PMOE_LOGITS_FEW
+  hipLaunchKernelGGL((router_logits_few_kernel<TW>), dim3(blocks_for(T, 16), blocks_for(E, 8)), dim3(128), 0, s, x, w, T,
+                     H, E, logits);
   return hipGetLastError();
 }
 template hipError_t router_logits_few<float>(const float*, const float*, int, int, int, float*, hipStream_t);

@@ -732,7 +732,7 @@ def _few_logits(x, W, K, **kw):
                                    (47, 1032, 33)])
 def test_router_fp32_few_experts(T, H, E):
     """fp32 rows at the edges of the few-expert logits kernel: 16 tokens a block,
-    8, 16 and 32 experts, H that its lanes share unevenly, and the GEMM beyond."""
+    8 experts a block, H that its lanes share unevenly, and the GEMM beyond 16."""
     say(f"fp32 router T={T} H={H} E={E}")
     g = gen(T + H)
     _few_logits(torch.randn(T, H, generator=g), torch.randn(E, H, generator=g) * 0.1, min(E, 3))
