@@ -32,6 +32,10 @@ hipError_t router_logits_gemm(const TX* x, const TW* w, int T, int H, int E, flo
 // The same from fp32 x for few experts: H a multiple of 4, x rows 16-byte and w rows 4-element aligned (route.hip).
 template <typename TW>
 hipError_t router_logits_few(const float* x, const TW* w, int T, int H, int E, float* logits, hipStream_t s);
+// The same for T <= 16 from bf16 x and an fp32 weight or its pieces [lo; hi; mid] (bf16): H a
+// multiple of 8, x and w 16-byte aligned (route.hip).
+template <typename TW>
+hipError_t router_logits_tokens(const bf16_t* x, const TW* w, int T, int H, int E, float* logits, hipStream_t s);
 // dx = dl . W   (dl: (T, ldl) fp32, columns >= E are ignored)
 template <typename TX, typename TW>
 hipError_t router_dx_gemm(const float* dl, int ldl, const TW* w, int T, int H, int E, TX* dx, hipStream_t s);

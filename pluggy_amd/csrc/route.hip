@@ -293,6 +293,62 @@ __global__ __launch_bounds__(128) void router_logits_few_kernel(const float* __r
     }
 }
 
+// The router weight of eight consecutive k, fp32 or as its bf16 pieces [lo; hi; mid]
+// n values apart, whose sum it is.
+__device__ __forceinline__ void load_w8(const float* w, int64_t, float (&v)[8]) {
+  const f32x4 a = load4(w), b = load4(w + 4);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) { v[i] = a[i]; v[4 + i] = b[i]; }
+}
+__device__ __forceinline__ void load_w8(const bf16_t* w, int64_t n, float (&v)[8]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const f32x4 lo = load4(w + 4 * h), hi = load4(w + n + 4 * h), mid = load4(w + 2 * n + 4 * h);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[4 * h + i] = (hi[i] + mid[i]) + lo[i];
+  }
+}
+
+// fp32 logits of few tokens (T <= TM) from bf16 rows and an fp32 weight: one
+// block per expert, each thread eight consecutive k of every 2048 for all
+// tokens, in fp32 FMAs of exact operands, summed over the wave and then over the
+// four waves. At these sizes the pass is latencies in a row: the GEMM on the
+// weight's bf16 pieces first writes and rereads them (a kernel and 2.5 MB at
+// 128 x 2048), then runs MFMA chains for mostly absent rows. Router forward at
+// H 2048, E 128, in a graph: one token 17.3 -> 8.5 us, 8 tokens 17.3 -> 10.9, 16
+// tokens 17.3 -> 13.6; H 2048, E 512, 16 tokens 24 -> 19.5.
+template <int TM, typename TW>
+__global__ __launch_bounds__(256) void router_logits_tokens_kernel(const bf16_t* __restrict__ x,
+                                                                  const TW* __restrict__ w, int T, int H, int E,
+                                                                  float* __restrict__ logits) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int e = blockIdx.x;
+  __shared__ float s_part[4][TM];
+  float acc[TM];
+#pragma unroll
+  for (int t = 0; t < TM; ++t) acc[t] = 0.0f;
+  for (int k = 8 * tid; k < H; k += 2048) {
+    float wv[8];
+    load_w8(w + (int64_t)e * H + k, (int64_t)E * H, wv);
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+      const bf16_t* xr = x + (int64_t)min(t, T - 1) * H + k;  // rows past the end repeat the last one
+      const f32x4 a = load4(xr), b = load4(xr + 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[t] = fmaf(a[i], wv[i], acc[t]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[t] = fmaf(b[i], wv[4 + i], acc[t]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < TM; ++t) {
+    const float v = wave_sum(acc[t]);
+    if (lane == 0) s_part[wave][t] = v;
+  }
+  __syncthreads();
+  if (tid < T) logits[(int64_t)tid * E + e] = (s_part[0][tid] + s_part[1][tid]) + (s_part[2][tid] + s_part[3][tid]);
+}
+
 // Router top-k with four rows per wave: each 16-lane DPP row of the wave takes
 // one token row, lane li holding experts li*V .. li*V+V-1 (E <= 16 V). The
 // same results as router_topk_kernel (logits, ids, top weights, statistics),
@@ -1207,6 +1263,23 @@ hipError_t router_logits_few(const float* x, const TW* w, int T, int H, int E, f
 }
 template hipError_t router_logits_few<float>(const float*, const float*, int, int, int, float*, hipStream_t);
 template hipError_t router_logits_few<bf16_t>(const float*, const bf16_t*, int, int, int, float*, hipStream_t);
+
+// H a multiple of 8; x and w 16-byte aligned. bf16 w: pieces [lo; hi; mid] of (E, H) each.
+template <typename TW>
+hipError_t router_logits_tokens(const bf16_t* x, const TW* w, int T, int H, int E, float* logits, hipStream_t s) {
+  if (T == 0) return hipSuccess;
+#define PMOE_LOGITS_TOK(TM) \
+  hipLaunchKernelGGL((router_logits_tokens_kernel<TM, TW>), dim3((unsigned)E), dim3(256), 0, s, x, w, T, H, E, logits)
+  if (T == 1) PMOE_LOGITS_TOK(1);
+  else if (T <= 4) PMOE_LOGITS_TOK(4);
+  else if (T <= 8) PMOE_LOGITS_TOK(8);
+  else if (T <= 16) PMOE_LOGITS_TOK(16);
+  else return hipErrorInvalidValue;
+#undef PMOE_LOGITS_TOK
+  return hipGetLastError();
+}
+template hipError_t router_logits_tokens<float>(const bf16_t*, const float*, int, int, int, float*, hipStream_t);
+template hipError_t router_logits_tokens<bf16_t>(const bf16_t*, const bf16_t*, int, int, int, float*, hipStream_t);
 
 template <typename TW>
 hipError_t router_topk(const float* parts, int nsplit, int64_t split_stride, int64_t ldp, float* logits,

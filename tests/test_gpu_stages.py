@@ -755,3 +755,6 @@ def test_router_few_tokens(T, H, E):
     assert odd.is_contiguous() and odd.data_ptr() % 16 == 4
     c = _ops().router_forward(x.to(DEV), odd, 4, True)
     assert rel(c[0], a[0].cpu().double()) < 1e-6 * max(H, 4) ** 0.5
+    bias = torch.randn(E, generator=g).to(DEV)
+    d = _ops().router_forward(x.to(DEV), W.to(DEV), 4, True, logit_bias=bias)
+    assert torch.equal(d[0], a[0] + bias)
