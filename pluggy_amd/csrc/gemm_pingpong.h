@@ -35,6 +35,12 @@
 
 namespace pmoe {
 
+// DMA instructions a wave may have in flight at a wait, two for each unit issued
+// after the one that has to have landed.
+constexpr int kPpFull = 12;     // six units
+constexpr int kPpFullHalf = 8;  // the same, two of the six being A1s not fetched for a next tile that is a half one
+constexpr int kPpHalf = 6;      // three units: of a half tile, and of a full one's last phase before a half one
+
 // 256 x 256 tiles of eight 128 x 64 wave tiles; wave row w holds rows 64 w ..
 // 64 w + 63 of both 128-row halves.
 template <typename Tc_>
@@ -325,17 +331,26 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     if (((tile + 2) & 31) == 0) fill_tiles(tile + 2, 32);
     // A tile's indices landed before the previous epilogue in the waves that fetched
-    // them; with two k tiles no phase's barrier lies between that and their use.
+    // them, and are read in k tile nk - 2: with two k tiles no phase's barrier lies
+    // between.
     if (GATH == GA_ROWS && nk == 2) lds_barrier();
     fetch_rows(tile + 2);
     if (second) swap_groups();
     // Phase P of k tile kt, whose DMAs fetch unit P of k tile lkt (two k tiles
-    // on). Ahead of a phase's end lie the units of the next six phases, two
-    // instructions each, so a wait for vmcnt(12) leaves the next phase's unit
-    // landed (8: two of the six may be A1s not fetched for a next tile that is
-    // a half one). A tile's first seven units landed before its first phase
-    // (the prologue, or the wait before the epilogue): no wait until phase 6,
-    // which gives the epilogue's stores, counted with the loads, six phases.
+    // on). Ahead of a phase's end lie the units of the next six phases, so a
+    // wait for kPpFull leaves the next phase's unit landed (kPpFullHalf: two of
+    // the six may be A1s not fetched for a next tile that is a half one).
+    //
+    // A wait covers the wave's own DMAs; a unit may be read once every wave has
+    // waited for its share and a barrier has followed. Every wave waits for all
+    // of the next tile's first two k tiles before its epilogue, but between that
+    // and the first group's first segment there is no barrier: what that
+    // segment reads has to have landed by the last phase's wait. That is A0
+    // (N0 is read already), and for a half tile N1 as well, hence kPpHalf in
+    // the last phase before one. The later units of those k tiles have the
+    // first segment's barrier behind them, so the tile waits for none before
+    // phase 6, which gives the epilogue's stores, counted with the loads, six
+    // phases.
     // The phases between the first two and the last k tiles (`lean`) check
     // none of that: their reads and DMAs are what a segment's length hangs on
     // (the checks there cost 6 to 10 % of the GEMMs' time).
@@ -352,10 +367,11 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
       else read_n(std::integral_constant<int, 0>());
       dma_unit(ld, pc, lean, lkt, par);
       if constexpr (LEAN) {
-        wait_vmcnt<12>();
+        wait_vmcnt<kPpFull>();
       } else if (kt > 1 || (P >= 2 && kt == 1)) {
-        if (few) wait_vmcnt<8>();
-        else wait_vmcnt<12>();
+        if (!few) wait_vmcnt<kPpFull>();
+        else if (P == 3 && kt == nk - 1) wait_vmcnt<kPpHalf>();
+        else wait_vmcnt<kPpFullHalf>();
       }
       __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0)
       swap_groups();
@@ -371,12 +387,12 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
     // A tile of at most 128 rows: two phases a k tile. The first reads A0 and N1,
     // the second the next N0, and they issue the units in the same order
     // (without its own A1s), so that tiles of both kinds follow each other.
-    // Three units at least follow the one each wait is for.
+    // Three units at least follow the last one each wait is for.
     auto half_k_tile = [&](int kt, int lkt) {
       read_a(std::integral_constant<int, 0>());
       read_n(std::integral_constant<int, 1>());
       dma_unit(ld, std::integral_constant<int, 0>(), kAny, lkt, par);
-      if (kt > 0) wait_vmcnt<6>();  // the next k tile's N0
+      if (kt > 0) wait_vmcnt<kPpHalf>();  // the next k tile's N0
       __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));
       swap_groups();
       mfmas(std::integral_constant<int, 0>());
@@ -385,7 +401,7 @@ __global__ __launch_bounds__(Cfg::NT, 1) void grouped_gemm_pp_kernel(GemmParams 
       for (int ks = 0; ks < 4; ++ks) lb[ks] ^= 2 * UNIT;
       read_n(std::integral_constant<int, 0>());
       static_for<1, 4>([&](auto uc) { dma_unit(ld, uc, kAny, lkt, par); });
-      if (kt > 0) wait_vmcnt<6>();  // its A0 and N1
+      if (kt > 0) wait_vmcnt<kPpHalf>();  // its A0 and N1
       __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));
       swap_groups();
       mfmas(std::integral_constant<int, 1>());

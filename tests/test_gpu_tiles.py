@@ -1,13 +1,14 @@
 """GPU: the row-grouped expert GEMMs at the edges of their tiles.
 
 Expert row counts on both sides of the tile (256 rows) and of its half (a tile
-of at most 128 rows runs half the matrix work), in sequences where both kinds
-follow each other on one block; reductions of one k tile, of an odd number and
-with a remainder; column counts that are not a multiple of the tile's. Gathered
-input rows and routing weights, every output against fp64 on the same 16-bit
-operands: an output is one rounding of an fp32 sum or of a short expression of
-such sums, so its relative error is about 2^-9 / sqrt(3) in bf16 (2^-12 /
-sqrt(3) in fp16), allowed three times over.
+of at most 128 rows runs half the matrix work); reductions of one k tile, of an
+odd number and with a remainder; column counts that are not a multiple of the
+tile's; and lists long enough that full and half tiles follow each other on a
+block (one block per CU walks the tiles). Gathered input rows and routing
+weights, every output against fp64 on the same 16-bit operands: an output is one
+rounding of an fp32 sum or of a short expression of such sums, so its relative
+error is about 2^-9 / sqrt(3) in bf16 (2^-12 / sqrt(3) in fp16), allowed three
+times over.
 """
 
 from __future__ import annotations
@@ -27,13 +28,13 @@ ROWS = {
 }
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("H, I", [(64, 32), (136, 72), (712, 264)])
-@pytest.mark.parametrize("rows", list(ROWS))
-def test_row_grouped_tile_edges(rows, H, I, dtype):
+# 11 tiles of both kinds (and an expert without rows) in eight experts
+CHAIN = [300, 100, 140, 520, 128, 257, 0, 60]
+
+
+def _check_rows(n, H, I, dtype):
     from pluggy_amd import ops
 
-    n = ROWS[rows]
     E, P = len(n), sum(n)
     say(f"tile edges {n} H={H} I={I} {dtype}")
     g = gen(11)
@@ -63,6 +64,45 @@ def test_row_grouped_tile_edges(rows, H, I, dtype):
     check_close("dw", part.sum(1, dtype=torch.float64), (dm * gate * s * up).sum(1), 1e-5, 1e-5)
     gx = ops.gate_up_dgrad(ggu, wgu.to(DEV), offs)
     check_close("dx_perm", gx, ref_grouped(ggu.cpu(), wgu, o, trans_w=False), tol, mx)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H, I", [(64, 32), (136, 72), (712, 264)])
+@pytest.mark.parametrize("rows", list(ROWS))
+def test_row_grouped_tile_edges(rows, H, I, dtype):
+    _check_rows(ROWS[rows], H, I, dtype)
+
+
+@pytest.mark.parametrize("H, I, dtype", [(1544, 1416, torch.bfloat16), (1544, 1416, torch.float16),
+                                         (72, 1416, torch.bfloat16), (1544, 72, torch.bfloat16)])
+def test_tiles_follow_each_other(H, I, dtype):
+    """88 m-tiles: two to four tiles a block in the GEMMs with many columns, at
+    23 to 45 k tiles, and at two (with and without gathered rows) and three."""
+    _check_rows(CHAIN * 8, H, I, dtype)
+
+
+def test_many_tiles_per_block():
+    """66 tiles a block (at 256 blocks) wrap the 64-entry ring of tile places.
+    Small integers: every output is exact."""
+    from pluggy_amd import ops
+
+    E, cols, K = 512, 8448, 8
+    n = [30, 38, 34, 140] * (E // 4)
+    P = sum(n)
+    say(f"ring of tile places: {E} experts, {P} rows, {cols} columns")
+    g = gen(3)
+    ints = lambda *s: torch.randint(-4, 5, s, generator=g).bfloat16().to(DEV)  # noqa: E731
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(n))[torch.randperm(P, generator=g)].reshape(-1, 1)
+    x, a, w = ints(P, K), ints(P, K), ints(E, cols, K)
+    _, offs, _, _, tok, sw = ops.permute_rows(ids.to(DEV), torch.ones(P, 1, device=DEV, dtype=torch.bfloat16), E)
+    y = ops.down_proj(a, w, offs)
+    gu, _ = ops.gate_up_swiglu(x, w, offs, tok, sw)
+    xs, lo = x[tok.long()], 0
+    for e, rows in enumerate(n):
+        we = w[e].float().t().contiguous()
+        assert torch.equal(y[lo:lo + rows].float(), a[lo:lo + rows].float() @ we), f"down_proj, expert {e}"
+        assert torch.equal(gu[lo:lo + rows].float(), xs[lo:lo + rows].float() @ we), f"gate_up, expert {e}"
+        lo += rows
 
 
 def _f32_case(rows, H, I, seed):
