@@ -1,25 +1,40 @@
 // fp32 expert GEMMs on the bf16 matrix cores.
 //
-// An fp32 value is the exact sum of three bf16 ones (8 + 8 + 8 significand
-// bits, by truncation: hi takes the top 8 bits, mid the next 8, lo the rest),
-// and a product of two bf16 values is exact in fp32. The six products hi.hi,
-// hi.mid, mid.hi, hi.lo, lo.hi and mid.mid hold everything down to 2^-22 of the
-// full product (what is left out, mid.lo + lo.mid + lo.lo, is about 2^-24 of
-// it), far below what fp32 accumulation over the reduction rounds away. bf16
-// MFMAs run 16 times as fast as fp32 ones on this chip, so six of them take
-// 3/8 of the time, and they round the accumulator six times per 16 k where
-// the fp32 ones (2 k each) round it eight times. Error against fp64 of the six
-// GEMMs at H 512, I 1024 and H 1024, I 512 (2048 tokens): 2.7e-7 to 7.2e-7, on
-// fp32 MFMAs 3.0e-7 to 8.1e-7. Time of the six together at the first shape 804
-// -> 522 us, at the second 1410 -> 788, 8192 tokens of the first 2425 -> 1479
-// (131 TFLOP/s of fp32 products at best, 790 of bf16 ones: like the large bf16
-// GEMMs, bound by the clock the chip can hold); these before the lane order of
-// SplitT, which took another 3 to 4 % off the whole pass.
+// An fp32 value is the exact sum of three bf16 ones, each the rounding (to
+// nearest) of what the ones before it left: mid is at most 2^-8 of hi's leading
+// power, lo 2^-17. A product of two bf16 values is exact in fp32. The six
+// products hi.hi, hi.mid, mid.hi, hi.lo, lo.hi and mid.mid are accumulated, the
+// smallest first; left out are mid.lo + lo.mid + lo.lo, at most 2^-24 of the
+// leading powers' product (half of an fp32 rounding), of random sign and 2^-27
+// of it typically. (With pieces by truncation, which cost the same, they reach
+// 2^-21 and always lie on one side.) bf16 MFMAs run 16 times as fast as fp32
+// ones on this chip, so six of them take 3/8 of the time, and they round the
+// accumulator six times per 16 k where the fp32 ones (2 k each) round it eight
+// times, though toward zero where those round to nearest.
 //
-// Infinities do not survive the split (inf times a zero piece is NaN): a tile
-// that meets one anywhere in its operands computes itself again with fp32
-// MFMAs. Pieces of values below 2^-102 may fall under bf16's normal range; the
-// product's error is then about 2^-126 times the other operand.
+// Relative error against fp64 of normally distributed operands, by the length n
+// of the reduction (on fp32 MFMAs): n 3 3.3e-8 (3.6e-8), 8 3.1e-8 (5.4e-8), 40
+// 8.3e-8 (1.15e-7), 128 1.6e-7 (2.0e-7), 512 3.4e-7 (4.1e-7), 2048 7.0e-7
+// (8.1e-7). Of one and two products it is 3.4e-8 (2.5e-8 and 3.0e-8), the
+// accumulator's rounding alone: tiles of at most kSplitMin reduction rows (an
+// expert's weight gradient from so few tokens) take fp32 MFMAs.
+//
+// Time of the six together at H 512, I 1024, 2048 tokens 804 -> 522 us, at H
+// 1024, I 512 1410 -> 788, 8192 tokens of the first 2425 -> 1479 (131 TFLOP/s of
+// fp32 products at best, 790 of bf16 ones: like the large bf16 GEMMs, bound by
+// the clock the chip can hold); these before the lane order of SplitT, which
+// took another 3 to 4 % off the whole pass.
+//
+// A tile with an operand that its pieces do not hold computes itself again on
+// fp32 MFMAs:
+//  * Infinities, NaNs and magnitudes that round to a bf16 infinity (from
+//    3.396e38) make a piece infinite or NaN, and every output they enter infinite
+//    or NaN with it: the accumulators say so, at the end.
+//  * bf16 subnormals, which the MFMAs take as they are, end at 2^-133, so below
+//    2^-110 bits may be lost. What the third piece is made from is then an fp32
+//    subnormal: one class comparison per value, which takes the place of the
+//    comparisons that found infinities among the operands (the fp32 forward and
+//    the six GEMMs measured the same within 1 %).
 #pragma once
 
 #include "gemm.h"
@@ -44,24 +59,26 @@ struct SplitCfg {
                 "the epilogue's slabs and the fp32 loop's stage fit");
 };
 
+// Reduction rows up to which a tile is computed on fp32 MFMAs alone.
+constexpr int kSplitMin = 3;
+constexpr int kSubnormal = 0x90, kNonFinite = 0x207;  // v_cmp_class_f32: +-subnormal; NaNs and +-infinity
+
 // Four consecutive k of one row, split: 8 bytes per plane.
 struct Split4 {
   uint32_t w[3][2];
+  bool inexact = false;  // a value's last piece may not hold all that is left of it
   __device__ __forceinline__ explicit Split4(const u32x4& v) {
-    float x[4], m[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[i] = __uint_as_float(v[i]);
-      m[i] = x[i] - __uint_as_float(v[i] & 0xffff0000u);
-    }
-    float l[4];
+    for (int h = 0; h < 2; ++h) {
+      float a = __uint_as_float(v[2 * h]), b = __uint_as_float(v[2 * h + 1]);  // what is left of two values
 #pragma unroll
-    for (int i = 0; i < 4; ++i) l[i] = m[i] - __uint_as_float(__float_as_uint(m[i]) & 0xffff0000u);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {  // the upper halves of two values
-      w[0][h] = __builtin_amdgcn_perm(v[2 * h + 1], v[2 * h], 0x07060302u);
-      w[1][h] = __builtin_amdgcn_perm(__float_as_uint(m[2 * h + 1]), __float_as_uint(m[2 * h]), 0x07060302u);
-      w[2][h] = __builtin_amdgcn_perm(__float_as_uint(l[2 * h + 1]), __float_as_uint(l[2 * h]), 0x07060302u);
+      for (int pl = 0; pl < 3; ++pl) {
+        if (pl == 2) inexact |= __builtin_amdgcn_classf(a, kSubnormal) | __builtin_amdgcn_classf(b, kSubnormal);
+        const uint32_t q = cvt_pk_bf16(a, b);
+        w[pl][h] = q;
+        a -= __uint_as_float(q << 16);
+        b -= __uint_as_float(q & 0xffff0000u);
+      }
     }
   }
   __device__ __forceinline__ void put(char* dst) const {  // dst: the row's chunk in plane 0
@@ -69,13 +86,6 @@ struct Split4 {
     for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<uint64_t*>(dst + pl * 64) = w[pl][0] | ((uint64_t)w[pl][1] << 32);
   }
 };
-
-// Largest magnitude among v's values and m (NaNs pass by: they stay NaN in the split).
-__device__ __forceinline__ float max_abs4(const u32x4& v, float m) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) m = __builtin_fmaxf(m, __builtin_fabsf(__uint_as_float(v[i])));
-  return m;
-}
 
 // Stagers: fp32 operand rows to LDS, as split planes (put) or as they are
 // (put_f32). R rows x 32 k, 256 threads.
@@ -98,13 +108,15 @@ struct SplitKc {  // k-contiguous: 8 chunks of 4 k per row
       reg[i] = v;
     }
   }
-  __device__ __forceinline__ float put(char* lds, int tid, float m) const {
+  __device__ __forceinline__ bool put(char* lds, int tid) const {
+    bool inexact = false;
 #pragma unroll
     for (int i = 0; i < PER_T; ++i) {
-      Split4(reg[i]).put(lds + ((tid + i * 256) >> 3) * SplitCfg::ROW + (tid & 7) * 8);
-      m = max_abs4(reg[i], m);
+      const Split4 sp(reg[i]);
+      sp.put(lds + ((tid + i * 256) >> 3) * SplitCfg::ROW + (tid & 7) * 8);
+      inexact |= sp.inexact;
     }
-    return m;
+    return inexact;
   }
   __device__ __forceinline__ void put_f32(float* lds, int tid) const {
 #pragma unroll
@@ -150,20 +162,21 @@ struct SplitT {  // [k][r]: 4 k-rows x 4 columns per unit
   __device__ __forceinline__ u32x4 row(int i, int c) const {
     return u32x4{reg[i][0][c], reg[i][1][c], reg[i][2][c], reg[i][3][c]};
   }
-  __device__ __forceinline__ float put(char* lds, int tid, float m) const {
+  __device__ __forceinline__ bool put(char* lds, int tid) const {
+    bool inexact = false;
 #pragma unroll
     for (int i = 0; i < PER_T; ++i) {
       const int u = tid + i * 256;
       if (UNITS % 256 == 0 || u < UNITS) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const u32x4 v = row(i, c);
-          Split4(v).put(lds + (col_of(u) + c) * SplitCfg::ROW + k_of(u) * 8);
-          m = max_abs4(v, m);
+          const Split4 sp(row(i, c));
+          sp.put(lds + (col_of(u) + c) * SplitCfg::ROW + k_of(u) * 8);
+          inexact |= sp.inexact;
         }
       }
     }
-    return m;
+    return inexact;
   }
   __device__ __forceinline__ void put_f32(float* lds, int tid) const {
 #pragma unroll
@@ -252,16 +265,18 @@ __global__ __launch_bounds__(SplitCfg::NT, 3) void grouped_gemm_split_kernel(Gem
 
   char* const ta = smem;
   char* const tb = smem + BM * ROW;
-  float mx = 0.0f;
-  if (nk > 0) {
+  // Short reductions and operands that the pieces do not hold go to fp32 MFMAs.
+  bool again = klen <= kSplitMin;
+  const int nsplit = again ? 0 : nk;
+  if (nsplit > 0) {
     sa.load(ti.k_lo, ti.k_hi, tid);
     sb.load(ti.k_lo, ti.k_hi, tid);
   }
-  for (int kt = 0; kt < nk; ++kt) {
-    mx = sa.put(ta, tid, mx);
-    mx = sb.put(tb, tid, mx);
+  for (int kt = 0; kt < nsplit; ++kt) {
+    again |= sa.put(ta, tid);
+    again |= sb.put(tb, tid);
     __syncthreads();
-    if (kt + 1 < nk) {  // the next stage's loads run under this one's MFMAs
+    if (kt + 1 < nsplit) {  // the next stage's loads run under this one's MFMAs
       sa.load(ti.k_lo + (kt + 1) * BK, ti.k_hi, tid);
       sb.load(ti.k_lo + (kt + 1) * BK, ti.k_hi, tid);
     }
@@ -290,8 +305,13 @@ __global__ __launch_bounds__(SplitCfg::NT, 3) void grouped_gemm_split_kernel(Gem
     }
     __syncthreads();
   }
-  if (__syncthreads_or(mx == __builtin_inff())) {
-    // an infinity among the operands: the same tile on fp32 MFMAs
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) again |= __builtin_amdgcn_classf(acc[i][j][r], kNonFinite);
+  if (__syncthreads_or(again)) {
     clear();
     float* const fa = reinterpret_cast<float*>(smem);
     float* const fb = fa + BM * Cfg::LDF;

@@ -16,7 +16,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from tests._gpu_helpers import DEV, MAX_ABS_FRAC, check_close, gen, ref_grouped, ref_wgrad, say
+from tests._gpu_helpers import DEV, MAX_ABS_FRAC, check_close, gen, ref_grouped, ref_wgrad, rel, say
 
 pytestmark = pytest.mark.gpu
 
@@ -125,8 +125,8 @@ def test_fp32_gemms_are_fp32_exact(H, I, scale):
     """fp32 operands through their bf16 pieces: the error against fp64 is that of
     fp32 sums. A sum of n products accumulated in fp32 in any order is off by at
     most n 2^-24 of the sum of magnitudes; roundings of random sign give about
-    sqrt(n) 2^-24 of the result's norm, allowed twice (the pieces left out, 2^-23
-    of a product at worst, are inside that)."""
+    sqrt(n) 2^-24 of the result's norm, allowed twice (the products of pieces left
+    out, 2^-24 of a product at worst and of random sign, are inside that)."""
     ops, x, wgu, wdn, offs, tok, sw = _f32_case([64, 65, 1, 0, 200, 63], H, I, 5)
     x = x * scale
     say(f"fp32 GEMMs H={H} I={I} scale={scale}")
@@ -142,6 +142,127 @@ def test_fp32_gemms_are_fp32_exact(H, I, scale):
     check_close("dx_perm", gx, ref_grouped(gg, wgu, o, trans_w=False), bound(2 * I), 1e-5)
     gw = ops.gate_up_wgrad(gg.to(DEV), wgu[0, :1].expand(x.shape[0], -1).contiguous().to(DEV), offs, len(wgu))
     check_close("dgate_up", gw, ref_wgrad(gg, wgu[0, :1].expand(x.shape[0], -1).contiguous(), o), bound(200), 1e-5)
+
+
+def _fma_chain(a, b):
+    """a^T b, (n, M) and (n, N), summed in fp32 one product after the other (each
+    product exact, one rounding per sum); in fp64."""
+    acc = torch.zeros(a.shape[1], b.shape[1], dtype=torch.float64)
+    for k in range(a.shape[0]):
+        acc = (acc + torch.outer(a[k].double(), b[k].double())).float().double()
+    return acc
+
+
+@pytest.mark.parametrize("same_sign", [False, True])
+def test_fp32_short_reductions(same_sign):
+    """Weight gradients of experts with few rows: no further from fp64 than a chain
+    of fp32 additions, in the norm (the same roundings drawn otherwise: 5 % of room)
+    and, where a single product is the sum, in every element (half an fp32 ulp)."""
+    from pluggy_amd import ops
+
+    rows = [1, 2, 3, 0, 4, 5, 8, 16, 31, 33, 64, 100]
+    offs = torch.tensor(rows).cumsum(0).int()
+    P, g = sum(rows), gen(21)
+    gg, x = torch.randn(P, 128, generator=g), torch.randn(P, 192, generator=g)
+    if same_sign:
+        gg, x = gg.abs(), x.abs()
+    say(f"fp32 short reductions, same sign: {same_sign}")
+    gw = ops.gate_up_wgrad(gg.to(DEV), x.to(DEV), offs.to(DEV), len(rows)).cpu().double()
+    ref = ref_wgrad(gg, x, offs)
+    lo = 0
+    for e, n in enumerate(rows):
+        if n:
+            chain = _fma_chain(gg[lo:lo + n], x[lo:lo + n])
+            r, c = rel(gw[e], ref[e]), rel(chain, ref[e])
+            say(f"  {n} rows: {r:.2e}, the chain's {c:.2e}")
+            assert r <= 1.05 * c
+        if n == 1:
+            assert (((gw[e] - ref[e]) / ref[e]).abs() <= 2.0 ** -24).all()
+        lo += n
+
+
+@pytest.mark.parametrize("n", [1, 8, 16])
+def test_fp32_products_of_full_pieces(n):
+    """Operands whose pieces are as large as they get, all of one sign, so that
+    whatever a product leaves out adds up. Up to 16 products are six MFMAs, of which
+    the last alone adds at the sum's magnitude (the others at 2^-7 of it), in one
+    step or in two of eight products: at most two fp32 ulps, 2^-22 (what products
+    of truncated pieces leave out reaches 2^-21)."""
+    from pluggy_amd import ops
+
+    bits = torch.tensor([0x3F80FFFF, 0x3F807FFF, 0x3F817F7F, 0x3F80FF7F, 0x3FFF7F7F], dtype=torch.int32)
+    v = bits.view(torch.float32).repeat(16)
+    a = v.repeat(n, 1)
+    say(f"fp32 products of full pieces, {n} rows")
+    offs = torch.tensor([n], dtype=torch.int32)
+    gw = ops.gate_up_wgrad(a.to(DEV), a.to(DEV), offs.to(DEV), 1).cpu().double()
+    ref = ref_wgrad(a, a, offs)
+    assert ((gw - ref).abs() <= 2.0 ** -22 * ref).all()
+
+
+def _six_f32_gemms(ops, x, wgu, wdn, offs, tok, A, G):
+    """name -> (output, fp64 reference) of the six GEMMs without routing weights: x (P, H) and
+    G (P, H) gathered by tok, A (P, I) in sorted rows; the input gradient's SwiGLU sees A in both
+    its halves."""
+    o, t, E = offs.cpu(), tok.cpu().long(), len(wgu)
+    d = lambda v: v.to(DEV)  # noqa: E731
+    aa = torch.cat([A, A], dim=1)
+    out = {"gate_up": (ops.gate_up_swiglu(d(x), d(wgu), offs, tok)[0], ref_grouped(x[t], wgu, o, trans_w=True)),
+           "down": (ops.down_proj(d(A), d(wdn), offs), ref_grouped(A, wdn, o, trans_w=True)),
+           "gate_up dgrad": (ops.gate_up_dgrad(d(aa), d(wgu), offs), ref_grouped(aa, wgu, o, trans_w=False)),
+           "gate_up wgrad": (ops.gate_up_wgrad(d(aa), d(x), offs, E, row_index=tok), ref_wgrad(aa, x[t], o)),
+           "down wgrad": (ops.down_proj_wgrad(d(G), d(A), offs, E, row_index=tok), ref_wgrad(G[t], A, o))}
+    gate = torch.linspace(-2.0, 2.0, A.shape[1]).expand(A.shape[0], -1)
+    dm, s = ref_grouped(G[t], wdn, o, trans_w=False), torch.sigmoid(gate.double())
+    out["down dgrad"] = (ops.down_proj_dgrad(d(G), d(torch.cat([gate, gate + 3.0], dim=1)), d(wdn), offs, tok)[0],
+                         torch.cat([dm * (gate + 3.0) * s * (1 + gate * (1 - s)), dm * gate * s], dim=1))
+    return out
+
+
+# of the operand rows and of the weights (and of the other operand of the weight
+# gradients): below bf16's range in the last piece, below fp32's normal range,
+# and where rounding to bf16 overflows
+@pytest.mark.parametrize("e1, e2", [(-108, 0), (-112, 0), (-122, 10), (-126, 30), (-138, 60), (127, -40)])
+def test_fp32_gemms_over_the_whole_range(e1, e2):
+    """Operands near the ends of fp32's range: the error of fp32 sums, as in
+    test_fp32_gemms_are_fp32_exact, in every GEMM."""
+    ops, x, wgu, wdn, offs, tok, _ = _f32_case([70, 0, 5, 45], 64, 40, 13)
+    g = gen(14)
+    far = lambda *s: ((torch.rand(s, generator=g, dtype=torch.float64) + 0.999) * 2.0 ** e1 *  # noqa: E731
+                      (torch.randint(0, 2, s, generator=g) * 2 - 1)).float()
+    x, A = far(*x.shape), far(x.shape[0], 40)
+    wgu, wdn = wgu * 2.0 ** e2, wdn * 2.0 ** e2
+    G = (torch.randn(x.shape, generator=g) * 2.0 ** e2)
+    say(f"fp32 GEMMs at 2^{e1} and 2^{e2}")
+    t, o, E = tok.cpu().long(), offs.cpu(), len(wgu)
+    aa = torch.cat([A, A], dim=1)
+    pairs = [(ops.gate_up_swiglu(x.to(DEV), wgu.to(DEV), offs, tok)[0], ref_grouped(x[t], wgu, o, trans_w=True), 64),
+             (ops.down_proj(A.to(DEV), wdn.to(DEV), offs), ref_grouped(A, wdn, o, trans_w=True), 40),
+             (ops.gate_up_dgrad(aa.to(DEV), wgu.to(DEV), offs), ref_grouped(aa, wgu, o, trans_w=False), 80),
+             (ops.gate_up_wgrad(torch.cat([G, G[:, :16]], 1).to(DEV), x.to(DEV), offs, E, row_index=tok),
+              ref_wgrad(torch.cat([G, G[:, :16]], 1), x[t], o), 70),
+             (ops.down_proj_wgrad(G.to(DEV), A.to(DEV), offs, E, row_index=tok), ref_wgrad(G[t], A, o), 70)]
+    for i, (got, ref, n) in enumerate(pairs):
+        check_close(f"{i}", got, ref, 2.0 * n ** 0.5 * 2.0 ** -24, 1e-5)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_fp32_gemms_confine_infinities(bad):
+    """One operand value that is no finite number: every output that it enters is
+    what fp32 arithmetic gives, every other one is itself, in all six GEMMs."""
+    ops, x, wgu, wdn, offs, tok, _ = _f32_case([70, 30], 64, 40, 9)
+    g = gen(10)
+    A, G = torch.randn(100, 40, generator=g), torch.randn(100, 64, generator=g)
+    x[17, 5], A[33, 7], G[61, 9] = bad, bad, bad
+    say(f"fp32 GEMMs with {bad}")
+    for name, (got, ref) in _six_f32_gemms(ops, x, wgu, wdn, offs, tok, A, G).items():
+        got, fine = got.cpu().double(), torch.isfinite(ref)
+        assert 0 < int((~fine).sum()) < ref.numel() // 4
+        assert torch.equal(fine, torch.isfinite(got)), name
+        if name != "down dgrad":  # (whose infinities meet the SwiGLU's factors)
+            assert torch.equal(torch.isnan(ref), torch.isnan(got)), name
+            assert torch.equal(ref[~fine].nan_to_num(nan=0.0), got[~fine].nan_to_num(nan=0.0)), name
+        check_close(name, got[fine], ref[fine], 2e-6, 1e-5)
 
 
 @pytest.mark.parametrize("bad", [float("inf"), -float("inf"), float("nan")])
