@@ -96,11 +96,27 @@ int router_logit_splits(int64_t T, int64_t H, int64_t E, bool pieces) {
 // (router_logits_few), of more from the row-tile GEMM: its time grows with E,
 // the GEMM's does not below 128. The router of 16 experts: 8192 tokens of H 1024
 // 56 -> 24 us, 16384 of H 2048 103 -> 54 (91 with a bf16 weight).
+// More than eight experts are two blocks, which both read x; a bf16 weight, whose
+// every load is converted, does not leave them the time once x (2^26 values, the
+// Infinity Cache's size) comes from HBM and the GEMM has blocks enough: 16
+// experts, bf16 weight, few / GEMM: 65536 tokens of H 1024 178 / 181 us, of H 2048
+// 401 / 326, of H 4096 729 / 615; 32768 of H 4096 276 / 314 (with an fp32 weight
+// 65536 of H 2048 298 / 328).
 constexpr int kRouterFewExperts = 16;
+bool router_few_experts(int64_t T, int64_t H, int64_t E, int w_dtype) {
+  return E <= kRouterFewExperts && (w_dtype == PMOE_F32 || E <= 8 || T <= 32768 || T * H <= (int64_t)1 << 26);
+}
 // Up to this many bf16 tokens take their logits from fp32 FMAs on the weight
 // itself (router_logits_tokens) instead of from its bf16 pieces' GEMM, whose time
 // hardly depends on the tokens below 128; at 16 the gain is down from 9 us to 4.
+// Where the caller gives the pieces, the GEMM has no split to wait for, and past
+// 2^26 products it is the faster: E 1024, H 8192, FMAs / GEMM: 9 tokens 41 / 43
+// us, 16 tokens 45 / 43; E 512, H 16384, 16 tokens 55 / 51; E 256, H 8192 24 /
+// 28.
 constexpr int kRouterFewTokens = 16;
+bool router_few_tokens(int64_t T, int64_t H, int64_t E, int w_dtype) {
+  return T <= kRouterFewTokens && (w_dtype == PMOE_F32 || T * H * E <= (int64_t)1 << 26);
+}
 int64_t router_splits(int64_t T) { return std::max<int64_t>(1, (T + kRouterSplitChunk - 1) / kRouterSplitChunk); }
 int64_t ldl_of(int64_t E) { return (E + 7) / 8 * 8; }
 
@@ -189,7 +205,7 @@ PMOE_API int pmoe_router_forward(const void* x, int x_dtype, const void* weight,
       lparts = parts;
       nsplit = splits;
       sstride = (int64_t)T * E;
-    } else if (pieces && t <= kRouterFewTokens && ((uintptr_t)x | (uintptr_t)weight) % 16 == 0) {
+    } else if (pieces && router_few_tokens(T, H, E, w_dtype) && ((uintptr_t)x | (uintptr_t)weight) % 16 == 0) {
       hipError_t st = w_dtype == PMOE_F32
                           ? router_logits_tokens<float>((const bf16_t*)x, (const float*)weight, t, h, e, logits, s)
                           : router_logits_tokens<bf16_t>((const bf16_t*)x, (const bf16_t*)weight, t, h, e, logits, s);
@@ -211,7 +227,7 @@ PMOE_API int pmoe_router_forward(const void* x, int x_dtype, const void* weight,
       nsplit = splits;
       sstride = (int64_t)T * E;
     } else {
-      const bool few = e <= kRouterFewExperts && ((uintptr_t)x | (uintptr_t)weight) % 16 == 0;
+      const bool few = router_few_experts(T, H, E, w_dtype) && ((uintptr_t)x | (uintptr_t)weight) % 16 == 0;
       hipError_t st = by_dtype(w_dtype, [&](auto wp) {
         typedef PMOE_ELEM(wp) W;
         if (few) return router_logits_few<W>((const float*)x, (const W*)weight, t, h, e, logits, s);

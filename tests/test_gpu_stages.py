@@ -758,3 +758,32 @@ def test_router_few_tokens(T, H, E):
     bias = torch.randn(E, generator=g).to(DEV)
     d = _ops().router_forward(x.to(DEV), W.to(DEV), 4, True, logit_bias=bias)
     assert torch.equal(d[0], a[0] + bias)
+
+
+@pytest.mark.parametrize("T,H,E", [(8, 8192, 1024), (9, 8192, 1024)])
+def test_router_few_tokens_with_pieces_of_a_large_weight(T, H, E):
+    """Both sides of the line between the few-token kernel and the GEMM on given
+    pieces (2^26 products); without pieces the kernel takes both."""
+    say(f"few-token router on pieces T={T} H={H} E={E}")
+    g = gen(T)
+    x = torch.randn(T, H, generator=g).bfloat16()
+    W = torch.randn(E, H, generator=g) * 0.1
+    a = _few_logits(x, W, 8)
+    b = _few_logits(x, W, 8, pieces=_ops().split_router_weight(W.to(DEV)))
+    if T * H * E <= 1 << 26:
+        assert all(torch.equal(u, v) for u, v in zip(a, b))
+    else:
+        assert rel(b[0], a[0].cpu().double()) < 1e-6 * H ** 0.5
+
+
+@pytest.mark.parametrize("T,H", [(32768, 2056), (65536, 1024), (65600, 1024)])
+def test_router_fp32_few_experts_bf16_weight(T, H):
+    """fp32 rows beside a bf16 weight, on both sides of the lines (32768 tokens, 2^26
+    values of x) past which nine to 16 experts go to the GEMM."""
+    say(f"fp32 router, bf16 weight T={T} H={H}")
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(T, H, generator=g, device=DEV)
+    W = (torch.randn(9, H, generator=g, device=DEV) * 0.1).bfloat16()
+    logits, _, _, _, counts, psum, _ = _ops().router_forward(x, W, 2, True)
+    assert rel(logits, x.double() @ W.double().t()) < 2.0 * H ** 0.5 * 2.0 ** -24
+    assert int(counts.sum()) == 2 * T and rel(psum.sum(), torch.tensor(float(T))) < 1e-5
