@@ -11,8 +11,9 @@
 // stored [k][m] / [k][n] and is transposed in registers while it is staged into
 // LDS. LDS tiles are always [row][k] so every MFMA fragment is one vector read.
 //
-// Compute types: bf16 (v_mfma_f32_32x32x16_bf16) and fp32
-// (v_mfma_f32_32x32x2_f32); both accumulate in fp32.
+// The kernel of this file (fp32, v_mfma_f32_32x32x2_f32) runs the fp32 router's
+// GEMMs: GM_NONE, and GM_RED in chunks of the reduction. Its parameters, tile
+// lookup and epilogue serve the other engines' kernels as well.
 #pragma once
 
 #include <type_traits>
@@ -28,20 +29,6 @@ enum GroupMode { GM_NONE = 0, GM_ROWS = 1, GM_RED = 2, GM_BATCH = 3 };
 enum EpiKind { EPI_STORE = 0, EPI_SWIGLU = 1, EPI_SWIGLU_BWD = 2, EPI_SUM3 = 3 };
 
 template <typename Tc> struct Mfma;
-
-template <> struct Mfma<bf16_t> {
-  static constexpr int KPACK = 8;  // consecutive k per lane in one fragment
-  static constexpr int MK = 16;    // k extent of one MFMA
-  static constexpr int BK = 64;    // k extent of one LDS stage (128 B per row)
-  static constexpr int PADK = 8;   // row padding (16 B) against bank conflicts
-  typedef bf16x8 frag_t;
-  __device__ static __forceinline__ frag_t load(const bf16_t* p) {
-    return *reinterpret_cast<const bf16x8*>(p);
-  }
-  __device__ static __forceinline__ f32x16 mma(frag_t a, frag_t b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-};
 
 template <> struct Mfma<float> {
   static constexpr int KPACK = 1;
@@ -77,9 +64,6 @@ struct TileCfg {
 
 // Element conversion of one 16-byte global chunk into LDS elements.
 template <typename Tg, typename Tc> struct ChunkCvt;
-template <> struct ChunkCvt<bf16_t, bf16_t> {
-  __device__ static __forceinline__ void put(bf16_t* dst, u32x4 v) { *reinterpret_cast<u32x4*>(dst) = v; }
-};
 template <> struct ChunkCvt<float, float> {
   __device__ static __forceinline__ void put(float* dst, u32x4 v) { *reinterpret_cast<u32x4*>(dst) = v; }
 };
@@ -135,20 +119,6 @@ struct KContigStager {
 // Transpose of one VEC x VEC register block: in[j] holds k = j, r = 0..VEC-1;
 // writes LDS row r with k = 0..VEC-1.
 template <typename Tg, typename Tc> struct BlockT;
-template <> struct BlockT<bf16_t, bf16_t> {
-  __device__ static __forceinline__ void put(bf16_t* dst, int ldk, const u32x4* in) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      u32x4 o;
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        uint32_t a = in[2 * p][c >> 1], b = in[2 * p + 1][c >> 1];
-        o[p] = (c & 1) ? ((a >> 16) | (b & 0xffff0000u)) : ((a & 0xffffu) | (b << 16));
-      }
-      *reinterpret_cast<u32x4*>(dst + c * ldk) = o;
-    }
-  }
-};
 template <> struct BlockT<bf16_t, float> {
   __device__ static __forceinline__ void put(float* dst, int ldk, const u32x4* in) {
 #pragma unroll
@@ -200,12 +170,10 @@ struct TransStager {
   const Tg* base;
   int64_t ld;
   int r0, r_hi;
-  const int32_t* kidx;  // k-row k is row kidx[k] of base (nullptr: row k)
   u32x4 reg[PER_T][VEC];
 
-  __device__ __forceinline__ void init(const Tg* base_, int64_t ld_, int r0_, int r_hi_,
-                                       const int32_t* kidx_ = nullptr) {
-    base = base_; ld = ld_; r0 = r0_; r_hi = r_hi_; kidx = kidx_;
+  __device__ __forceinline__ void init(const Tg* base_, int64_t ld_, int r0_, int r_hi_) {
+    base = base_; ld = ld_; r0 = r0_; r_hi = r_hi_;
   }
   __device__ __forceinline__ void load(int k0, int k_hi, int tid) {
 #pragma unroll
@@ -219,7 +187,7 @@ struct TransStager {
         int k = k0 + kb * VEC + j;
         u32x4 v = {0u, 0u, 0u, 0u};
         if (ok_r && k < k_hi) {
-          const Tg* src = base + (int64_t)(kidx != nullptr ? kidx[k] : k) * ld + r;
+          const Tg* src = base + (int64_t)k * ld + r;
           if (r + VEC <= r_hi) v = *reinterpret_cast<const u32x4*>(src);
           else v = load_partial16(src, r_hi - r);
         }
@@ -419,19 +387,16 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[Cfg::MI][Cfg::NI]
 
 // ----------------------------------------------------------------- kernel ----
 
-template <class Cfg, typename TA, typename TB, typename Tout, bool A_KC, bool B_KC, int GM, int EPI>
+template <class Cfg, typename TA, typename TB, typename Tout, bool A_KC, bool B_KC, int GM>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_kernel(GemmParams p) {
   typedef typename Cfg::Tc Tc;
   typedef Mfma<Tc> MF;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, LDK = Cfg::LDK, NT = Cfg::NT;
   constexpr int MI = Cfg::MI, NI = Cfg::NI;
+  static_assert(GM == GM_NONE || GM == GM_RED, "the fp32 router's GEMMs");
   static_assert(!(GM == GM_RED && (A_KC || B_KC)), "GM_RED expects [k][m] and [k][n] operands");
-  static_assert(EPI != EPI_SWIGLU || (B_KC && GM == GM_ROWS), "SwiGLU epilogue is the gate_up forward");
-  static_assert(EPI != EPI_SWIGLU || (Cfg::NI % 2 == 0), "SwiGLU pairs gate and up halves of a wave tile");
 
   __shared__ __attribute__((aligned(16))) char smem[Cfg::SMEM_BYTES];
-  __shared__ int s_scan[1025];
-  __shared__ int s_found;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -439,35 +404,25 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_kernel(GemmParams p) {
   const int wm = wave / Cfg::WAVES_N, wn = wave % Cfg::WAVES_N;
 
   // ---- tile mapping
-  const int ntiles_n = (EPI == EPI_SWIGLU) ? (p.inter + BN / 2 - 1) / (BN / 2) : (p.N + BN - 1) / BN;
+  const int ntiles_n = (p.N + BN - 1) / BN;
   const int bid = blockIdx.x;
   const int tn = bid % ntiles_n;
   const int slot = bid / ntiles_n;
   TileInfo ti;
   const TA* A = reinterpret_cast<const TA*>(p.A);
   const TB* B = reinterpret_cast<const TB*>(p.B);
-  if constexpr (GM == GM_ROWS) {
-    int g, r0, re;
-    if (!rows_tile_lookup<BM>(p.offs, p.groups, slot, s_scan, &s_found, g, r0, re)) return;
-    ti.group = g; ti.m0 = r0; ti.m_end = re; ti.k_lo = 0; ti.k_hi = p.K;
-    B += (int64_t)g * p.strideB;
-  } else if constexpr (GM == GM_RED) {
+  if constexpr (GM == GM_RED) {
     const int mt = (p.M + BM - 1) / BM;
     const int g = slot / mt;
     if (g >= p.groups) return;
     ti.group = g; ti.m0 = (slot % mt) * BM; ti.m_end = p.M;
-    if (p.offs != nullptr) {
-      ti.k_lo = g == 0 ? 0 : p.offs[g - 1];
-      ti.k_hi = p.offs[g];
-    } else {
-      ti.k_lo = g * p.split_chunk;
-      ti.k_hi = min(p.K, ti.k_lo + p.split_chunk);
-    }
+    ti.k_lo = g * p.split_chunk;
+    ti.k_hi = min(p.K, ti.k_lo + p.split_chunk);
   } else {
     ti.group = 0; ti.m0 = slot * BM; ti.m_end = p.M; ti.k_lo = 0; ti.k_hi = p.K;
     if (ti.m0 >= p.M) return;
   }
-  ti.n0 = (EPI == EPI_SWIGLU) ? tn * (BN / 2) : tn * BN;
+  ti.n0 = tn * BN;
 
   // LDS stage s holds the A tile at [s*STAGE_ELEMS] and the B tile right after it.
   // Addresses are always formed from the __shared__ base so they stay in the
@@ -484,31 +439,16 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_kernel(GemmParams p) {
   if constexpr (A_KC) {
     const int m0 = ti.m0, me = ti.m_end;
     const int64_t lda = p.lda;
-    const int32_t* ai = p.a_index;
-    sa.init([&](int r) -> const TA* {
-      return (m0 + r < me) ? A + (int64_t)(ai != nullptr ? ai[m0 + r] : m0 + r) * lda : nullptr;
-    }, tid);
+    sa.init([&](int r) -> const TA* { return (m0 + r < me) ? A + (int64_t)(m0 + r) * lda : nullptr; }, tid);
   } else {
-    sa.init(A, p.lda, ti.m0, ti.m_end, p.a_index);
+    sa.init(A, p.lda, ti.m0, ti.m_end);
   }
   if constexpr (B_KC) {
-    const int n0 = ti.n0, N = p.N, I = p.inter;
+    const int n0 = ti.n0, N = p.N;
     const int64_t ldb = p.ldb;
-    if constexpr (EPI == EPI_SWIGLU) {
-      // Block column c -> B row: each wave's WN columns are WN/2 gate rows then
-      // the WN/2 matching up rows (offset I), so one lane holds both halves.
-      sb.init([&](int c) -> const TB* {
-        int w = c / Cfg::WN, cc = c % Cfg::WN, h = Cfg::WN / 2;
-        int gcol = n0 + w * h + (cc % h);
-        if (gcol >= I) return nullptr;
-        int row = (cc < h) ? gcol : I + gcol;
-        return B + (int64_t)row * ldb;
-      }, tid);
-    } else {
-      sb.init([&](int c) -> const TB* { return (n0 + c < N) ? B + (int64_t)(n0 + c) * ldb : nullptr; }, tid);
-    }
+    sb.init([&](int c) -> const TB* { return (n0 + c < N) ? B + (int64_t)(n0 + c) * ldb : nullptr; }, tid);
   } else {
-    sb.init(B, p.ldb, ti.n0, p.N, p.b_index);
+    sb.init(B, p.ldb, ti.n0, p.N);
   }
 
   f32x16 acc[MI][NI];
@@ -560,7 +500,7 @@ __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_kernel(GemmParams p) {
   }
 
   // ---- epilogue: stage each 32-row slab of the wave tile through LDS as fp32
-  store_tile<Cfg, Tout, GM, EPI>(acc, reinterpret_cast<float*>(smem), ti, p, wave, wm, wn, lane);
+  store_tile<Cfg, Tout, GM, EPI_STORE>(acc, reinterpret_cast<float*>(smem), ti, p, wave, wm, wn, lane);
 }
 
 // ------------------------------------------------------------- launchers ----
@@ -584,17 +524,16 @@ inline GemmParams zero_params() {
   return p;
 }
 
-template <class Cfg, typename TA, typename TB, typename Tout, bool A_KC, bool B_KC, int GM, int EPI>
+template <class Cfg, typename TA, typename TB, typename Tout, bool A_KC, bool B_KC, int GM>
 hipError_t launch_gemm(const GemmParams& p, hipStream_t s) {
-  const int ntn = (EPI == EPI_SWIGLU) ? (p.inter + Cfg::BN / 2 - 1) / (Cfg::BN / 2) : (p.N + Cfg::BN - 1) / Cfg::BN;
+  const int ntn = (p.N + Cfg::BN - 1) / Cfg::BN;
   int64_t slots;
-  if (GM == GM_ROWS) slots = (p.M + Cfg::BM - 1) / Cfg::BM + p.groups;
-  else if (GM == GM_RED) slots = (int64_t)p.groups * ((p.M + Cfg::BM - 1) / Cfg::BM);
+  if (GM == GM_RED) slots = (int64_t)p.groups * ((p.M + Cfg::BM - 1) / Cfg::BM);
   else slots = (p.M + Cfg::BM - 1) / Cfg::BM;
   const int64_t grid = slots * ntn;
   if (grid <= 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((grouped_gemm_kernel<Cfg, TA, TB, Tout, A_KC, B_KC, GM, EPI>), dim3((unsigned)grid),
+  hipLaunchKernelGGL((grouped_gemm_kernel<Cfg, TA, TB, Tout, A_KC, B_KC, GM>), dim3((unsigned)grid),
                      dim3(Cfg::NT), 0, s, p);
   return hipGetLastError();
 }

@@ -158,7 +158,7 @@ hipError_t router_logits_gemm(const TX* x, const TW* w, int T, int H, int E, flo
   p.B = w; p.ldb = H;
   p.C = logits; p.ldc = E;
   p.M = T; p.N = E; p.K = H;
-  return launch_gemm<CfgF32, TX, TW, float, true, true, GM_NONE, EPI_STORE>(p, s);
+  return launch_gemm<CfgF32, TX, TW, float, true, true, GM_NONE>(p, s);
 }
 
 // Router GEMM tile configurations. The logits GEMM from the three bf16 pieces
@@ -279,7 +279,7 @@ hipError_t router_dx_gemm(const float* dl, int ldl, const TW* w, int T, int H, i
   p.B = w; p.ldb = H;  // B[k=e][n=h] = W[e][h]
   p.C = dx; p.ldc = H;
   p.M = T; p.N = H; p.K = E;
-  return launch_gemm<CfgF32, float, TW, TX, true, false, GM_NONE, EPI_STORE>(p, s);
+  return launch_gemm<CfgF32, float, TW, TX, true, false, GM_NONE>(p, s);
 }
 
 template <typename TX>
@@ -291,20 +291,16 @@ hipError_t router_dw_gemm(const float* dl, int ldl, const TX* x, int T, int H, i
   p.C = partial; p.ldc = H; p.strideC = (int64_t)E * H;
   p.offs = nullptr; p.split_chunk = split_chunk; p.groups = (T + split_chunk - 1) / split_chunk;
   p.M = E; p.N = H; p.K = T;
-  return launch_gemm<CfgF32, float, TX, float, false, false, GM_RED, EPI_STORE>(p, s);
+  return launch_gemm<CfgF32, float, TX, float, false, false, GM_RED>(p, s);
 }
 
 #define PMOE_INST_ROUTER(TX, TW)                                                                              \
   template hipError_t router_logits_gemm<TX, TW>(const TX*, const TW*, int, int, int, float*, hipStream_t);  \
   template hipError_t router_dx_gemm<TX, TW>(const float*, int, const TW*, int, int, int, TX*, hipStream_t);
 
-PMOE_INST_ROUTER(bf16_t, float)
-PMOE_INST_ROUTER(bf16_t, bf16_t)
 PMOE_INST_ROUTER(float, float)
 PMOE_INST_ROUTER(float, bf16_t)
 
-template hipError_t router_dw_gemm<bf16_t>(const float*, int, const bf16_t*, int, int, int, int, float*,
-                                           hipStream_t);
 template hipError_t router_dw_gemm<float>(const float*, int, const float*, int, int, int, int, float*,
                                           hipStream_t);
 
