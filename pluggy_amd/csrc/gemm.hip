@@ -24,7 +24,8 @@ typedef TileCfg<float, 64, 128, 32, 64> CfgF32;
 // the next tile's first three stages are then in flight before a tile's
 // epilogue stores, which drain while they are used. The row-grouped GEMMs
 // (forward and input gradients) take the same tiles in the ping-pong loop of
-// gemm_pingpong.h: on this engine's loop they measured, alternating launches
+// gemm_pingpong.h, except for the shortest reductions (short_plain): on this
+// engine's loop they measured, alternating launches
 // at 8192 tokens, gate_up 507 against 472 us, down 289 / 262, down's input
 // gradient 306 / 280, gate_up's 472 / 430; at the Qwen3-235B-A22B layer and
 // 16384 tokens 3270 / 3050, 1674 / 1560, 1801 / 1610, 3022 / 2810. The weight
@@ -33,11 +34,11 @@ typedef TileCfg<float, 64, 128, 32, 64> CfgF32;
 // operands: 512-byte ones), so they stay here.
 typedef DmaCfg<256, 256, 128, 64, 4, 32, 1> DmaExpert;
 // Row-grouped GEMMs whose 256-row tiles would leave whole rounds of the
-// persistent walk idle: 128 x 256 blocks of eight 64 x 64 wave tiles (same
-// ring and k order, so the same bits). A 128-row tile moves 3/4 of a 256-row
-// tile's bytes per stage and, the k-loop being bound by those bytes, takes
-// ≈0.75 of its time (measured 0.70-0.77 on one GPU's EP=8 share of config 2),
-// so it pays only where it keeps the number of rounds: see use_rows128.
+// persistent walk idle: 128 x 256 blocks of eight 64 x 64 wave tiles (the same
+// k order, so the same bits). A 128-row tile moves 3/4 of the bytes per stage of
+// this engine's 256-row tile and took 0.70-0.77 of its time (one GPU's EP=8
+// share of config 2), so it pays only where it keeps the number of rounds: see
+// use_rows128.
 typedef DmaCfg<128, 256, 64, 64, 4, 32, 1> DmaExpert128;
 // The router's input gradient: one tile per CU, so no epilogue to hide; the
 // three-stage ring as measured.
@@ -91,6 +92,15 @@ int num_cus() {
 // dgrad (3 column tiles) fits one round either way and takes 0.75 of the
 // time, while gate_up fwd (6) would need two rounds instead of one; configs
 // 2-4 keep 256-row tiles throughout.
+// Against the ping-pong loop's 256-row tiles, whose half tiles the estimate does
+// not know, where the rule takes 128 (128 / 256 rows, H 2048, I 768): 8 experts of
+// 256 rows gate_up fwd 35 / 44 us, down fwd 17 / 22, down dgrad 32 / 48, gate_up
+// dgrad 24 / 36; 16 of 512 down dgrad 40 / 53; 32 of 600 down dgrad 95 / 116. It is
+// wrong where the 256-row tiles just fit one round and it expects two: 8 of 900
+// down fwd 36 / 30, 16 of 440 down fwd 36 / 31 and gate_up dgrad 53 / 49, 32 of 240
+// gate_up fwd 90 / 62. Over 266 such GEMMs of three layers 128 rows are the faster
+// by 1.08 (gate_up fwd), 1.13 (down fwd), 1.32 (down dgrad) and 1.22 (gate_up
+// dgrad).
 bool use_rows128(int kind, int P, int E, int H, int I, int cus) {
   if (kind == EG_DOWN_WGRAD || kind == EG_GATE_UP_WGRAD || E <= 0 || P < 128 * E) return false;
   const int ntn = kind == EG_GATE_UP_FWD ? (I + 127) / 128 : (kind == EG_DOWN_DGRAD ? (I + 255) / 256 : (H + 255) / 256);
@@ -100,6 +110,20 @@ bool use_rows128(int kind, int P, int E, int H, int I, int cus) {
     return std::ceil(tiles / cus);
   };
   return 0.75 * rounds(128) < rounds(256);
+}
+
+// Whether a row-grouped GEMM without a fused epilogue stays on the persistent
+// engine's own loop although its tiles have 256 rows: a reduction of at most two
+// of the ping-pong loop's 64-deep k tiles, of which it always runs two and waits
+// for both before the first product, while the persistent loop starts on the
+// first 32-deep stage. H 128, I 64, 64 experts of 520 rows: down 13.4 (ping-pong)
+// and 10.5 us, gate_up's input gradient 13.5 and 11.9; 32 experts of 2000 rows:
+// 20.5 and 16.0, 21.3 and 18.6. At H = I = 256 (reductions of 256 and 512) the two
+// loops are even on the whole (1.00 and 1.04 of each other over 17 sizes). With a
+// fused epilogue the ping-pong loop is not slower at a reduction of 128 either.
+constexpr int kShortReduction = 128;
+bool short_plain(int kind, int H, int I) {
+  return (kind == EG_DOWN_FWD && I <= kShortReduction) || (kind == EG_GATE_UP_DGRAD && 2 * I <= kShortReduction);
 }
 
 }  // namespace
@@ -125,6 +149,8 @@ hipError_t expert_gemm_run(int kind, const T* A, const T* B, const T* aux, T* C,
     if (rows == Cfgs::Rows128::BM)
       return expert_gemm_persist_rows<typename Cfgs::Rows128>(kind, A, B, aux, C, C2, offs, P, E, H, I, xg, num_cus(),
                                                                s);
+    if (short_plain(kind, H, I))
+      return expert_gemm_persist_plain<typename Cfgs::Main>(kind, A, B, C, offs, P, E, H, I, num_cus(), s);
     if (!wgrad)
       return expert_gemm_pp_rows<PpCfg<T>>(kind, A, B, aux, C, C2, offs, P, E, H, I, xg, num_cus(), s);
     return expert_gemm_persist_wgrad<typename Cfgs::Main, Tw>(kind, A, B, Cw, offs, P, E, H, I, xg, num_cus(), s);

@@ -583,9 +583,11 @@ __device__ __forceinline__ bool deal_below_mean(const unsigned short* s_order, i
 // The tile list of a persistent kernel and this block's tiles of it.
 //
 // XCD x (blocks with blockIdx % 8 == x) takes a contiguous share of the tiles
-// and its blocks walk it in a stride of their count. GM_ROWS tiles all run
-// the full reduction, so the shares hold equal tile counts; a GM_RED tile
-// runs its group's reduction range, so there the shares hold equal cost.
+// and its blocks walk it in a stride of their count. GM_ROWS shares hold equal
+// tile counts, since their tiles all run the full reduction (those of at most
+// 128 rows in half the phases in the ping-pong loop, which this does not
+// weigh); a GM_RED tile runs its group's reduction range, so there the shares
+// hold equal cost.
 // Under skewed routing (GM_RED, one tile costing more than half a block's
 // mean share) the shares cannot balance: a heavy group's tiles crowd one
 // XCD's blocks. Then the tiles are taken in order of descending cost and
@@ -1160,6 +1162,17 @@ hipError_t expert_gemm_persist_rows(int kind, const T16* A, const T16* B, const 
       return launch_gemm_persist<Cfg, true, false, GM_ROWS, EPI_SWIGLU_BWD>(p, num_cus, s);
     case EG_GATE_UP_DGRAD: return launch_gemm_persist<Cfg, true, false, GM_ROWS, EPI_STORE>(p, num_cus, s);
   }
+  return hipErrorInvalidValue;
+}
+
+// The row-grouped GEMMs without a fused epilogue (down forward, gate_up dgrad)
+// on the persistent kernel.
+template <class Cfg, typename T16 = typename Cfg::Tc>
+hipError_t expert_gemm_persist_plain(int kind, const T16* A, const T16* B, T16* C, const int32_t* offs, int P, int E,
+                                     int H, int I, int num_cus, hipStream_t s) {
+  const GemmParams p = expert_params<T16>(kind, A, B, nullptr, C, nullptr, offs, P, E, H, I);
+  if (kind == EG_DOWN_FWD) return launch_gemm_persist<Cfg, true, true, GM_ROWS, EPI_STORE>(p, num_cus, s);
+  if (kind == EG_GATE_UP_DGRAD) return launch_gemm_persist<Cfg, true, false, GM_ROWS, EPI_STORE>(p, num_cus, s);
   return hipErrorInvalidValue;
 }
 

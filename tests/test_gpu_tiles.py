@@ -77,32 +77,43 @@ def test_row_grouped_tile_edges(rows, H, I, dtype):
                                          (72, 1416, torch.bfloat16), (1544, 72, torch.bfloat16)])
 def test_tiles_follow_each_other(H, I, dtype):
     """88 m-tiles: two to four tiles a block in the GEMMs with many columns, at
-    23 to 45 k tiles, and at two (with and without gathered rows) and three."""
+    23 to 45 k tiles, at two (of gathered rows) and at three."""
     _check_rows(CHAIN * 8, H, I, dtype)
 
 
 def test_many_tiles_per_block():
-    """66 tiles a block (at 256 blocks) wrap the 64-entry ring of tile places.
-    Small integers: every output is exact."""
+    """66 tiles a block (at 256 blocks) wrap the 64-entry ring of tile places, without
+    gathered rows at three k tiles and with them at two. Signs and zeros: every
+    output is a whole number of at most 136, exact in bf16."""
     from pluggy_amd import ops
 
-    E, cols, K = 512, 8448, 8
+    E, cols = 512, 8448
     n = [30, 38, 34, 140] * (E // 4)
     P = sum(n)
     say(f"ring of tile places: {E} experts, {P} rows, {cols} columns")
-    g = gen(3)
-    ints = lambda *s: torch.randint(-4, 5, s, generator=g).bfloat16().to(DEV)  # noqa: E731
+    g, gd = gen(3), torch.Generator(device=DEV).manual_seed(3)
+    signs = lambda *s: torch.randint(-1, 2, s, generator=gd, device=DEV).bfloat16()  # noqa: E731
     ids = torch.repeat_interleave(torch.arange(E), torch.tensor(n))[torch.randperm(P, generator=g)].reshape(-1, 1)
-    x, a, w = ints(P, K), ints(P, K), ints(E, cols, K)
     _, offs, _, _, tok, sw = ops.permute_rows(ids.to(DEV), torch.ones(P, 1, device=DEV, dtype=torch.bfloat16), E)
-    y = ops.down_proj(a, w, offs)
-    gu, _ = ops.gate_up_swiglu(x, w, offs, tok, sw)
-    xs, lo = x[tok.long()], 0
-    for e, rows in enumerate(n):
-        we = w[e].float().t().contiguous()
-        assert torch.equal(y[lo:lo + rows].float(), a[lo:lo + rows].float() @ we), f"down_proj, expert {e}"
-        assert torch.equal(gu[lo:lo + rows].float(), xs[lo:lo + rows].float() @ we), f"gate_up, expert {e}"
-        lo += rows
+    for name, K in (("down_proj", 136), ("gate_up", 8)):
+        x, w = signs(P, K), signs(E, cols, K)
+        if name == "down_proj":
+            y, xs = ops.down_proj(x, w, offs), x
+        else:
+            y, xs = ops.gate_up_swiglu(x, w, offs, tok, sw)[0], x[tok.long()]
+        lo = 0
+        for e, rows in enumerate(n):
+            ref = xs[lo:lo + rows].float() @ w[e].float().t().contiguous()
+            assert torch.equal(y[lo:lo + rows].float(), ref), f"{name}, expert {e}"
+            lo += rows
+
+
+@pytest.mark.parametrize("I", [56, 64, 72, 128, 136])
+def test_short_reductions_of_plain_gemms(I):
+    """Both sides of the reduction of 128 up to which down's forward and gate_up's
+    input gradient keep the persistent engine's loop: the same sums either way,
+    over full and half tiles."""
+    _check_rows(CHAIN, 264, I, torch.bfloat16)
 
 
 def _f32_case(rows, H, I, seed):
