@@ -314,9 +314,11 @@ __device__ __forceinline__ void load_w8(const bf16_t* w, int64_t n, float (&v)[8
 // tokens, in fp32 FMAs of exact operands, summed over the wave and then over the
 // four waves. At these sizes the pass is latencies in a row: the GEMM on the
 // weight's bf16 pieces first writes and rereads them (a kernel and 2.5 MB at
-// 128 x 2048), then runs MFMA chains for mostly absent rows. Router forward at
-// H 2048, E 128, in a graph: one token 17.3 -> 8.5 us, 8 tokens 17.3 -> 10.9, 16
-// tokens 17.3 -> 13.6; H 2048, E 512, 16 tokens 24 -> 19.5.
+// 128 x 2048) unless the caller has them, then runs MFMA chains for mostly absent
+// rows. Router forward at H 2048, E 128, in a graph: one token 17.3 -> 8.8 us, 8
+// tokens 17.2 -> 11.0, 16 tokens 17.4 -> 13.7; H 2048, E 512, 16 tokens 24 ->
+// 19.7. On given pieces (six bytes a weight instead of four) 15.1 -> 8.7, 11.1 and
+// 14.0, and 20.6 -> 20.0.
 template <int TM, typename TW>
 __global__ __launch_bounds__(256) void router_logits_tokens_kernel(const bf16_t* __restrict__ x,
                                                                   const TW* __restrict__ w, int T, int H, int E,
