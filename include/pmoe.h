@@ -333,7 +333,7 @@ PMOE_API int pmoe_expert_ffn_backward(const void* grad_out, const void* hidden, 
  * tile the grouped-GEMM engine gives an expert GEMM, for tests and tuning.
  * kind: PMOE_GEMM_* below; dtype: the operands' (PMOE_BF16 and PMOE_F16 take the
  * persistent DMA engine: 32-row tiles for the forward GEMMs of few-token
- * batches, 128 or 256 otherwise; PMOE_F32 the register-staged one: 64 rows);
+ * batches, 128 or 256 otherwise; PMOE_F32 the one that splits fp32 operands: 64 rows);
  * num_cus <= 0: the current device's compute units. Returns the tile's rows,
  * or a negative PMOE_ERR_* code. Host-only: launches nothing. */
 enum {
